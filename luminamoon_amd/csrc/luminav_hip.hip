@@ -150,9 +150,9 @@ static bool same_class(const Item &x, const Item &y) {
     return x.pass == y.pass && x.step == y.step && x.pt == y.pt && x.gt == y.gt && x.st == y.st && x.master == y.master;
 }
 
-static int launch_one(KernelFn fn, const Args &args, uint32_t grid, uint32_t threads, hipStream_t stream) {
+static int launch_one(KernelFn fn, const Args &args, uint32_t grid, uint32_t threads, hipStream_t stream, uint32_t lds = 0) {
     void *kargs[] = {const_cast<Args *>(&args)};
-    hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(fn), dim3(grid), dim3(threads), kargs, 0, stream);
+    hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(fn), dim3(grid), dim3(threads), kargs, lds, stream);
     if (e != hipSuccess) return fail(LV_STATUS_EXECUTION_FAILED, "kernel launch failed: %s", hipGetErrorString(e));
     return LV_STATUS_SUCCESS;
 }
@@ -161,8 +161,8 @@ static uint64_t units_of(uint64_t n, uint32_t unit_elems) { return (n + unit_ele
 
 // Count slots a tensor of `units` work units takes in a table launch: its count slots and its fold
 // slot.
-static uint64_t table_slots_of(uint64_t units) {
-    return (uint64_t)table_count_slots(units > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)units) + 1;
+static uint64_t table_slots_of(uint64_t units, uint32_t unit_elems) {
+    return (uint64_t)launch_count_slots(units > 0xFFFFFFF0ull ? 0xFFFFFFF0u : (uint32_t)units, unit_elems, true) + 1;
 }
 
 static int dtype_bytes(int dt) { return dt == LV_DTYPE_F32 ? 4 : 2; }
@@ -319,8 +319,8 @@ static Layout make_layout(char *ws, uint64_t table_slots, uint32_t radial_units)
 
 // What a call needs, from its tensors alone (an upper bound over every class the call forms):
 // table count slots when more than kMaxDesc tensors step, and radial unit records up to one piece
-// when the config uses the radial bound. Units are counted at the smallest unit size of table and
-// radial launches, 1024 elements (the one-wave blocks of unit_threads are inline launches only).
+// when the config uses the radial bound. Units are counted at 1024 elements, the smallest unit size of
+// radial launches and the one that table launches' count slots follow (launch_count_slots).
 static void call_needs(const lv_config *cfg, const lv_tensor *T, int count, uint64_t &table_slots, uint32_t &radial_units) {
     table_slots = 0;
     radial_units = 0;
@@ -333,7 +333,7 @@ static void call_needs(const lv_config *cfg, const lv_tensor *T, int count, uint
         active++;
         const uint64_t u = units_of(T[i].numel, kHalf);
         units += u;
-        slots += table_slots_of(u);
+        slots += table_slots_of(u, kHalf);
     }
     if (active > kMaxDesc && !radial) table_slots = slots;
     if (radial) radial_units = (uint32_t)std::min<uint64_t>(units, kRadialPiece);
@@ -583,7 +583,7 @@ static int launch(Args &args, int mode, int pt, int st, int pass, hipStream_t st
     // slower. Results are the same either way: units are independent and the count is exact in
     // any order.
     const bool identity_map = st == LV_DTYPE_F32 && !radial &&
-                              (lv::unit_threads(mode, pt, st, pass, args.flags, table) < kThreads ||
+                              (unit_threads(mode, pt, st, pass, args.flags, table) < kThreads ||
                                args.total_units <= kIdentityMapUnits);
     args.xcds = identity_map ? 1u : device_xcds();
     // b / X == (b * recip) >> 40 for b < 2^23 = kMaxGrid and X <= 64: recip exceeds 2^40 / X by at
@@ -603,13 +603,16 @@ static int launch(Args &args, int mode, int pt, int st, int pass, hipStream_t st
     }
     if (max_grid == 0) return fail(LV_STATUS_INVALID_CONFIG, "no radial unit records in the workspace");
     KernelFn fold = radial ? pick_fold(mode, pass) : nullptr;
+    const uint32_t threads = unit_threads(mode, pt, st, pass, args.flags, table);
+    // one-wave blocks of a large launch: as many per CU as HBM streams best with (wave_resident)
+    const uint32_t lds = (args.flags & kFWave) ? wave_lds_bytes(wave_resident(mode, pt, (args.flags & kFMaster) != 0, table)) : 0u;
     for (uint32_t ub = 0; ub < args.total_units; ub += std::min<uint32_t>(max_grid, args.total_units - ub)) {
         const uint32_t grid = std::min<uint32_t>(max_grid, args.total_units - ub);
         args.unit_base = ub;
         args.piece_units = grid;
         args.xcd_q = grid / args.xcds;
         args.xcd_r = grid % args.xcds;
-        int rc = launch_one(fn, args, grid, lv::unit_threads(mode, pt, st, pass, args.flags, table), stream);
+        int rc = launch_one(fn, args, grid, threads, stream, lds);
         if (rc != LV_STATUS_SUCCESS) return rc;
         if (radial) {
             uint32_t chunks = 0;
@@ -716,7 +719,14 @@ static uint64_t desc_units(const Desc &D, uint32_t unit_elems) {
     return units_of(D.n - (D.vec ? D.head : 0u), unit_elems);
 }
 
-static void fill_args_common(Args &args, const lv_config *cfg, const Item &h, int bound) {
+// kWaveElems, or LV_WAVE_ELEMS (so tests can run the one-wave kernels of large launches on small ones).
+static uint64_t wave_elems() {
+    const char *e = std::getenv("LV_WAVE_ELEMS");
+    return e ? std::strtoull(e, nullptr, 10) : kWaveElems;
+}
+
+// `elems`: the elements of the launch's class.
+static void fill_args_common(Args &args, const lv_config *cfg, const Item &h, int bound, uint64_t elems, bool table) {
     std::memset(&args, 0, sizeof args);
     args.lr = cfg->lr;
     args.b1 = cfg->beta1;
@@ -754,6 +764,7 @@ static void fill_args_common(Args &args, const lv_config *cfg, const Item &h, in
     if (bound == LV_BOUND_COORDINATE) flags |= kFCoordinate;
     if (bound == LV_BOUND_RADIAL) flags |= kFRadial;
     flags |= (uint32_t)h.gt << 8;
+    if (elems >= wave_elems() && unit_wave(cfg->buffer, h.pt, h.st, h.pass, flags, table)) flags |= kFWave;
     args.flags = flags;
 }
 
@@ -830,10 +841,12 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
         while (cls_end < nitems && same_class(items[cls_end], h)) cls_end++;
         const bool radial = bound == LV_BOUND_RADIAL && h.pass != kSingle;
         const bool table = !radial && L.table_slots > 0 && tab_buf && cls_end - begin > kMaxDesc;
+        uint64_t elems = 0;
+        for (int k = begin; k < cls_end; k++) elems += tensors[items[k].idx].numel;
         if (table) {
             const int n = cls_end - begin;
             Args args;
-            fill_args_common(args, cfg, h, bound);
+            fill_args_common(args, cfg, h, bound, elems, table);
             args.step_rec = rec;
             const uint32_t unit_elems = lv::unit_elems(cfg->buffer, h.pt, h.st, h.pass, args.flags, true);
             std::vector<TDesc> &tab = *tab_buf;
@@ -850,7 +863,7 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
                 if (units > 0xFFFFFFFFull) return fail(LV_STATUS_INVALID_CONFIG, "too many work units in one launch");
                 E.unit_end = (uint32_t)units;
                 E.slot_base = (uint32_t)slot;
-                slot += table_slots_of(u);
+                slot += table_slots_of(u, unit_elems);
             }
             if (slot > L.table_slots)
                 return fail(LV_STATUS_INVALID_CONFIG, "workspace too small: %llu table count slots needed, %llu present",
@@ -876,7 +889,7 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
         while (begin < cls_end) {
             const int end = begin + std::min(cls_end - begin, kMaxDesc);
             Args args;
-            fill_args_common(args, cfg, h, bound);
+            fill_args_common(args, cfg, h, bound, elems, table);
             args.step_rec = rec;
             const uint32_t unit_elems = lv::unit_elems(cfg->buffer, h.pt, h.st, h.pass, args.flags, false);
             args.ndesc = end - begin;

@@ -65,6 +65,7 @@ enum Pass : int { kSingle = 0, kFused = 1, kCount = 2, kApply = 3 };
 
 enum Flags : uint32_t {
     kFDynamic = 1u << 31,  // template flag set: read the flags from the launch arguments
+    kFWave = 1u << 30,     // template flag set: this word's kernel in one-wave blocks (wave_resident)
     kFCautious = 1u << 0,
     kFSR = 1u << 1,
     kFMaster = 1u << 2,
@@ -101,16 +102,67 @@ constexpr int unit_min_blocks(int mode, int pt, int st, int pass, uint32_t flags
     return unit_subs(mode, pt, st, pass, flags) > 1 ? 8 : 1;
 }
 
+// Resident one-wave blocks per CU of a large f32-state launch, 0 where it keeps 256-thread blocks.
+//
+// The f32-state steps are bound by HBM, and HBM's rate depends on how many waves stream at once. A
+// full CU (32 waves) puts more requests in flight than the memory system keeps in order, and the
+// same kernel over the same buffers runs faster with fewer waves resident, down to where too few
+// bytes are in flight (the rate then falls off steeply). One-wave blocks on 256-element units, held
+// to the number below by unused dynamic LDS (wave_lds_bytes), measured against 256-thread blocks (8
+// per CU; CLM f32 and T2 bf16 inline: one-wave blocks, 32 per CU), interleaved in one process on the
+// same buffers, 1.2e8 (f32) and 9.5e8 (16-bit params) elements:
+//
+//   step (state f32)             before, us   blocks per CU: us
+//   CLM  f32, table                  580.4    32: 562.3   21: 545.9   18: 534.1   16: 545.2   14: 569.7
+//   CLM  f32, bucket                 555.1    32: 554.4   21: 536.7   18: 529.3   16: 534.7   14: 550.9
+//   T2   f32, table                  615.7    32: 574.5   21: 548.8   18: 543.2   16: 540.8   14: 529.6
+//   TD   f32, table                  400.5    32: 394.7   25: 388.8   21: 379.6   18: 392.9   16: 408.0
+//   T1   f32, table                  400.7    32: 387.5   21: 381.4   18: 377.1   16: 378.4   14: 396.3
+//   T2   bf16, table                3407.6    32: 3238.6  21: 3186.2  18: 3196.0  16: 3311.0  14: 3579.8
+//   T2   bf16, bucket of 3.5e9     12320      32: 12369   21: 12129   18: 11919   16: 12091
+//   T2   f16, table                 3624.3    32: 3291.7  25: 3265.9  21: 3304.0  18: 3422.9
+//   CLM  bf16 + master, table       4644.2    32: 4309.8  25: 4239.9  21: 4168.1  18: 4228.6
+//   T1   bf16 + master, table       3003.6    32: 3002.5  21: 2895.0  18: 2866.6  16: 2952.4
+//   TD   bf16 + master, table       3219.2    32: 2960.2  25: 2925.7  21: 3008.5
+//   T2   bf16 + master, table       4527.7    32: 4578.4  18: 4424.9  16: 4310.9  14: 4213.7
+//   T2   f16 + master, table        4600.4    32: 4430.2  18: 4270.8  16: 4148.9  14: 4197.2
+//
+// More arithmetic per byte needs more waves, more bytes per wave fewer. T1 with 16-bit params and no
+// master moves too few bytes per wave for a limit (table 2152 -> 2071 at 32 per CU, 2163 at 25; its
+// inline launches stay level with 256-thread blocks, 2069). CLM and TD-CLM with 16-bit params and no
+// master are bound by their arithmetic: CLM f16 4143 -> 4167, TD bf16 2336 -> 2331 at 32 per CU.
+constexpr uint32_t wave_resident(int mode, int pt, bool master, bool table) {
+    if (pt == LV_DTYPE_F32)
+        return mode == LV_BUFFER_T2 ? 16u : mode == LV_BUFFER_TDCLM ? 21u : 18u;
+    if (master) return mode == LV_BUFFER_TDCLM ? 25u : mode == LV_BUFFER_DUAL ? 21u : mode == LV_BUFFER_T1 ? 18u : 16u;
+    if (mode == LV_BUFFER_T2) return pt == LV_DTYPE_BF16 ? 18u : 25u;
+    return mode == LV_BUFFER_T1 && table ? 32u : 0u;
+}
+
+// Dynamic LDS bytes of a one-wave block that leave room for `resident` blocks on a CU: LDS is 160 KB
+// in granules of 1280 bytes, and the kernel's own few bytes stay within the last granule.
+constexpr uint32_t wave_lds_bytes(uint32_t resident) { return resident && resident < 32u ? 128u / resident * 1280u - 256u : 0u; }
+
+// Smallest launch (elements of its class) that takes the one-wave kernels of wave_resident. Below it
+// a CU sees each of its waves only a few times and the limit costs what the order gains: at 4e6
+// elements 0.91-1.02x, at 8e6 0.97-1.02x, at 1.6e7 0.99-1.03x, at 3.2e7 1.01-1.05x (CLM f32, T2 bf16).
+constexpr uint64_t kWaveElems = 1ull << 25;
+
+// Whether the kernels of this word have a one-wave form (kFWave): the steady pass with f32 state and
+// the reference defaults, with or without a master copy.
+constexpr bool unit_wave(int mode, int pt, int st, int pass, uint32_t flags, bool table) {
+    return st == LV_DTYPE_F32 && pass == kFused && (flags & ~(uint32_t)(kFMaster | kFWave)) == static_flags(pt, pass) &&
+           wave_resident(mode, pt, (flags & kFMaster) != 0, table) != 0;
+}
+
 // Threads per block of the unit kernel for this mode, dtypes, pass, flag word (the launch's word;
-// the run-time-flag kernels have 256) and launch kind. Two steady inline steps with f32 state and
-// the reference defaults run one-wave blocks (units of 256 elements), which launch() maps block b
-// to unit b. In one process on the same buffers, against 256-thread blocks:
+// the run-time-flag kernels have 256) and launch kind. The kFWave kernels run one-wave blocks (units
+// of 256 elements), and so do two steady inline steps with f32 state and the reference defaults at
+// every size. In one process on the same buffers, against 256-thread blocks:
 // - CLM in f32 (cfg3's kernel): 0.938-0.966x (cfg3, and a 1e9-element bucket);
-// - T2 with bf16 params (the headline's kernel): 0.966x at 1e9 elements, 0.959x at 3.5e9, and
-//   0.992-1.005x at cfg5's 6.7e9 (five processes).
-// The other kernels keep 256: T1 with f32 state ran 1.040-1.046x with one-wave blocks (cfg4),
-// TD-CLM's table launch of 64 tensors (cfg2) 1.03x (its inline buckets 0.980-0.986x).
+// - T2 with bf16 params (the headline's kernel): 0.966x at 1e9 elements, 0.959x at 3.5e9.
 constexpr int unit_threads(int mode, int pt, int st, int pass, uint32_t flags, bool table) {
+    if (flags & kFWave) return 64;
     const bool one_wave = (mode == LV_BUFFER_DUAL && pt == LV_DTYPE_F32) || (mode == LV_BUFFER_T2 && pt == LV_DTYPE_BF16);
     return (!table && one_wave && st == LV_DTYPE_F32 && pass == kFused && flags == static_flags(pt, pass)) ? 64 : kThreads;
 }
@@ -165,6 +217,14 @@ __host__ __device__ inline uint32_t table_count_slots(uint32_t units) {
     if (c <= 1u) return 1u;
     if (c >= kSlots) return kSlots;
     return 1u << (32 - __builtin_clz(c - 1u));
+}
+
+// Count slots of a tensor of `units` work units of `unit_elems` elements in a launch. One-wave table
+// launches keep the slot count of 1024-element units (the workspace is sized for those): their slots
+// see up to 256 blocks.
+__host__ __device__ inline uint32_t launch_count_slots(uint32_t units, uint32_t unit_elems, bool table) {
+    const uint32_t r = table && unit_elems < kHalf ? kHalf / unit_elems : 1u;
+    return table_count_slots((units + r - 1u) / r);
 }
 
 // Radial-bound sums of a run of units: sum u_eff^2, sum p^2 (f64), mask count.
@@ -1451,7 +1511,8 @@ __device__ __forceinline__ int find_tensor(const Args &a, uint32_t unit) {
 // Counting unit launches: thread 0 of every block reports its exact mask count and the block's
 // completion in ONE 64-bit atomic (count << kTicketBits | 1) on one of the tensor's S count slots
 // (slot = unit index in the tensor mod S, 64 B apart, so the atomics spread over L2 channels;
-// S = table_count_slots(units): the smallest power of two keeping every slot at <= 64 blocks, at
+// S = launch_count_slots: the smallest power of two keeping every slot at <= 64 blocks (256 one-wave
+// blocks of a table launch), at
 // most 64). The block whose report completes a slot (its ticket reaches the slot's block count)
 // holds that slot's whole count in the value its own atomic returned and re-zeroes the slot; a
 // tensor of one slot (<= 64 units) is then complete, and that block finalises the scratch. With
@@ -1461,13 +1522,13 @@ __device__ __forceinline__ int find_tensor(const Args &a, uint32_t unit) {
 // returned by an atomic on that same word, so no fence is needed (a device-scope release fence
 // per block measured 7x slower); integer sums are exact in any order, so the result is
 // deterministic. Wholly inactive units report a zero count.
-template <int MODE, int PASS, bool TABLE>
+template <int MODE, int PASS, bool TABLE, uint32_t UNIT>
 __device__ __forceinline__ void report_count(const Args &a, const Desc &D, const View &tv, uint32_t unit,
                                              uint32_t count) {
     const uint32_t n_units = tv.t_end - tv.t_begin;
     const uint32_t k = unit - tv.t_begin;
     // slot s of S takes units k = s (mod S): n_units / S blocks, plus one for s < n_units % S
-    const uint32_t S = table_count_slots(n_units);  // a power of two, <= 64 blocks per slot
+    const uint32_t S = launch_count_slots(n_units, UNIT, TABLE);  // a power of two
     const uint32_t s = k & (S - 1u);
     const uint32_t nslots = n_units < S ? n_units : S;
     unsigned long long *words = a.slots + (size_t)tv.slot_base * kSlotStride;
@@ -1557,7 +1618,7 @@ __global__ void __launch_bounds__(unit_threads(MODE, PT, ST, PASS, FL, TABLE), u
     constexpr int TPB = unit_threads(MODE, PT, ST, PASS, FL, TABLE);  // threads per block
     __shared__ BlockSums<TPB> sh;
 
-    const uint32_t flags = (FL & kFDynamic) ? a.flags : FL;
+    const uint32_t flags = (FL & kFDynamic) ? a.flags : (FL & ~(uint32_t)kFWave);
     const bool radial = kCounting && (flags & kFRadial);  // squared norms summed in this pass
     // Workgroups are dispatched to the XCDs round-robin (block b runs on XCD b mod X). Map them so
     // that each XCD streams one contiguous range of units, or, where the host passes X = 1, block
@@ -1697,7 +1758,7 @@ __global__ void __launch_bounds__(unit_threads(MODE, PT, ST, PASS, FL, TABLE), u
                 uint32_t tot = 0;
 #pragma unroll
                 for (int k = 0; k < TPB / 64; k++) tot += (uint32_t)sh.cnt[k];
-                report_count<MODE, PASS, TABLE>(a, D, tv, unit, tot);
+                report_count<MODE, PASS, TABLE, (uint32_t)kUnit>(a, D, tv, unit, tot);
             }
         }
     }
@@ -1832,6 +1893,17 @@ template <int MODE, int PT, int ST, int PASS>
 KernelFn pick_flags(uint32_t flags, bool table) {
     constexpr uint32_t kStatic = static_flags(PT, PASS);
     constexpr uint32_t kRadial = radial_flags(PT);
+    if constexpr (PASS == kFused && ST == LV_DTYPE_F32) {  // the one-wave kernels of large launches
+        constexpr uint32_t kW = kStatic | kFWave, kWM = kW | kFMaster;
+        if (flags == kW) {
+            if constexpr (unit_wave(MODE, PT, ST, PASS, kW, true))
+                if (table) return unit_kernel<MODE, PT, ST, PASS, kW, true>;
+            if constexpr (unit_wave(MODE, PT, ST, PASS, kW, false))
+                if (!table) return unit_kernel<MODE, PT, ST, PASS, kW, false>;
+        }
+        if constexpr (PT != LV_DTYPE_F32 && unit_wave(MODE, PT, ST, PASS, kWM, true))
+            if (flags == kWM) return table ? unit_kernel<MODE, PT, ST, PASS, kWM, true> : unit_kernel<MODE, PT, ST, PASS, kWM, false>;
+    }
     if (table) {
         if (flags == kStatic) return unit_kernel<MODE, PT, ST, PASS, kStatic, true>;
         return unit_kernel<MODE, PT, ST, PASS, kFDynamic, true>;
