@@ -605,7 +605,7 @@ static int launch(Args &args, int mode, int pt, int st, int pass, hipStream_t st
     KernelFn fold = radial ? pick_fold(mode, pass) : nullptr;
     const uint32_t threads = unit_threads(mode, pt, st, pass, args.flags, table);
     // one-wave blocks of a large launch: as many per CU as HBM streams best with (wave_resident)
-    const uint32_t lds = (args.flags & kFWave) ? wave_lds_bytes(wave_resident(mode, pt, (args.flags & kFMaster) != 0, table)) : 0u;
+    const uint32_t lds = threads < kThreads && (args.flags & kFLarge) ? wave_lds_bytes(wave_resident(mode, pt, (args.flags & kFMaster) != 0, table)) : 0u;
     for (uint32_t ub = 0; ub < args.total_units; ub += std::min<uint32_t>(max_grid, args.total_units - ub)) {
         const uint32_t grid = std::min<uint32_t>(max_grid, args.total_units - ub);
         args.unit_base = ub;
@@ -719,10 +719,10 @@ static uint64_t desc_units(const Desc &D, uint32_t unit_elems) {
     return units_of(D.n - (D.vec ? D.head : 0u), unit_elems);
 }
 
-// kWaveElems, or LV_WAVE_ELEMS (so tests can run the one-wave kernels of large launches on small ones).
-static uint64_t wave_elems() {
-    const char *e = std::getenv("LV_WAVE_ELEMS");
-    return e ? std::strtoull(e, nullptr, 10) : kWaveElems;
+// kLargeElems, or LV_LARGE_ELEMS (so tests can run the kernels of large launches on small ones).
+static uint64_t large_elems() {
+    const char *e = std::getenv("LV_LARGE_ELEMS");
+    return e ? std::strtoull(e, nullptr, 10) : kLargeElems;
 }
 
 // `elems`: the elements of the launch's class.
@@ -764,19 +764,11 @@ static void fill_args_common(Args &args, const lv_config *cfg, const Item &h, in
     if (bound == LV_BOUND_COORDINATE) flags |= kFCoordinate;
     if (bound == LV_BOUND_RADIAL) flags |= kFRadial;
     flags |= (uint32_t)h.gt << 8;
-    if (elems >= wave_elems() && unit_wave(cfg->buffer, h.pt, h.st, h.pass, flags, table)) flags |= kFWave;
+    // A counting pass without the radial bound reads neither the rounding, the decay, the bound nor the
+    // master options: it takes the kernel of the reference defaults.
+    if (h.pass == kCount && bound != LV_BOUND_RADIAL && cfg->cautious && h.gt == h.pt) flags = static_flags(h.pt, kCount);
+    if (elems >= large_elems() && unit_large(cfg->buffer, h.pt, h.st, h.pass, flags, table)) flags |= kFLarge;
     args.flags = flags;
-}
-
-// The launches of one class (or of one inline group of at most kMaxDesc tensors of it).
-static int launch_class(Args &args, const lv_config *cfg, const Item &h, hipStream_t stream, bool table,
-                        uint32_t radial_piece) {
-    if (h.pass == kCount) {
-        int rc = launch(args, cfg->buffer, h.pt, h.st, kCount, stream, table, radial_piece);
-        if (rc != LV_STATUS_SUCCESS) return rc;
-        return launch(args, cfg->buffer, h.pt, h.st, kApply, stream, table, radial_piece);
-    }
-    return launch(args, cfg->buffer, h.pt, h.st, h.pass, stream, table, radial_piece);
 }
 
 // An item's step count and first pass: dual.rs:52, dual.rs:122, dual.rs:260; tdclm.rs:67-68.
@@ -843,12 +835,17 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
         const bool table = !radial && L.table_slots > 0 && tab_buf && cls_end - begin > kMaxDesc;
         uint64_t elems = 0;
         for (int k = begin; k < cls_end; k++) elems += tensors[items[k].idx].numel;
-        if (table) {
+        // A two-pass class runs its counting pass, then the applying pass, each with work units of its
+        // own kernel's size.
+        Item ph = h;  // the class, with the pass being launched
+        const int npass = h.pass == kCount ? 2 : 1;
+        for (int pi = 0; table && pi < npass; pi++) {
+            ph.pass = pi == 0 ? h.pass : (int)kApply;
             const int n = cls_end - begin;
             Args args;
-            fill_args_common(args, cfg, h, bound, elems, table);
+            fill_args_common(args, cfg, ph, bound, elems, table);
             args.step_rec = rec;
-            const uint32_t unit_elems = lv::unit_elems(cfg->buffer, h.pt, h.st, h.pass, args.flags, true);
+            const uint32_t unit_elems = lv::unit_elems(cfg->buffer, ph.pt, ph.st, ph.pass, args.flags, true);
             std::vector<TDesc> &tab = *tab_buf;
             if (tab.size() < (size_t)n) tab.resize((size_t)n);
             uint64_t units = 0, slot = 0;
@@ -879,42 +876,47 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
             int rc = acquire_table(tab.data(), (size_t)n, stream, lease);
             if (rc != LV_STATUS_SUCCESS) return rc;
             args.dtab = lease.s->dev;
-            rc = launch_class(args, cfg, h, stream, true, 0);
+            rc = launch(args, cfg->buffer, ph.pt, ph.st, ph.pass, stream, true, 0);
             const int rr = release_table(lease, stream);
             if (rc != LV_STATUS_SUCCESS) return rc;
             if (rr != LV_STATUS_SUCCESS) return rr;
+        }
+        if (table) {
             begin = cls_end;
             continue;
         }
         while (begin < cls_end) {
             const int end = begin + std::min(cls_end - begin, kMaxDesc);
-            Args args;
-            fill_args_common(args, cfg, h, bound, elems, table);
-            args.step_rec = rec;
-            const uint32_t unit_elems = lv::unit_elems(cfg->buffer, h.pt, h.st, h.pass, args.flags, false);
-            args.ndesc = end - begin;
-            uint64_t units = 0;
-            for (int k = begin; k < end; k++) {
-                Desc &D = args.d[k - begin];
-                const lv_tensor &T = tensors[items[k].idx];
-                fill_desc(D, T, items[k], dual, unit_elems);
-                D.unit_begin = (uint32_t)units;
-                units += desc_units(D, unit_elems);
-                if (units > 0xFFFFFFFFull) return fail(LV_STATUS_INVALID_CONFIG, "too many work units in one launch");
+            for (int pi = 0; pi < npass; pi++) {
+                ph.pass = pi == 0 ? h.pass : (int)kApply;
+                Args args;
+                fill_args_common(args, cfg, ph, bound, elems, table);
+                args.step_rec = rec;
+                const uint32_t unit_elems = lv::unit_elems(cfg->buffer, ph.pt, ph.st, ph.pass, args.flags, false);
+                args.ndesc = end - begin;
+                uint64_t units = 0;
+                for (int k = begin; k < end; k++) {
+                    Desc &D = args.d[k - begin];
+                    const lv_tensor &T = tensors[items[k].idx];
+                    fill_desc(D, T, items[k], dual, unit_elems);
+                    D.unit_begin = (uint32_t)units;
+                    units += desc_units(D, unit_elems);
+                    if (units > 0xFFFFFFFFull) return fail(LV_STATUS_INVALID_CONFIG, "too many work units in one launch");
+                }
+                args.total_units = (uint32_t)units;
+                if (radial && units > L.radial_units && !L.radial_split)
+                    return fail(LV_STATUS_INVALID_CONFIG,
+                                "radial launch of %llu work units exceeds the %u unit records of this entry point",
+                                (unsigned long long)units, L.radial_units);
+                args.slots = L.slots;
+                args.tickets = L.tickets;
+                args.run = L.run;
+                args.chunks = L.chunks;
+                args.unit_sq = L.unit_sq;
+                args.unit_cnt = L.unit_cnt;
+                const int rc = launch(args, cfg->buffer, ph.pt, ph.st, ph.pass, stream, false, L.radial_units);
+                if (rc != LV_STATUS_SUCCESS) return rc;
             }
-            args.total_units = (uint32_t)units;
-            if (radial && units > L.radial_units && !L.radial_split)
-                return fail(LV_STATUS_INVALID_CONFIG,
-                            "radial launch of %llu work units exceeds the %u unit records of this entry point",
-                            (unsigned long long)units, L.radial_units);
-            args.slots = L.slots;
-            args.tickets = L.tickets;
-            args.run = L.run;
-            args.chunks = L.chunks;
-            args.unit_sq = L.unit_sq;
-            args.unit_cnt = L.unit_cnt;
-            const int rc = launch_class(args, cfg, h, stream, false, L.radial_units);
-            if (rc != LV_STATUS_SUCCESS) return rc;
             begin = end;
         }
     }

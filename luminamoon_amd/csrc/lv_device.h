@@ -65,7 +65,7 @@ enum Pass : int { kSingle = 0, kFused = 1, kCount = 2, kApply = 3 };
 
 enum Flags : uint32_t {
     kFDynamic = 1u << 31,  // template flag set: read the flags from the launch arguments
-    kFWave = 1u << 30,     // template flag set: this word's kernel in one-wave blocks (wave_resident)
+    kFLarge = 1u << 30,    // template flag set: this word's kernel in its form for large launches (unit_large)
     kFCautious = 1u << 0,
     kFSR = 1u << 1,
     kFMaster = 1u << 2,
@@ -90,8 +90,13 @@ constexpr uint32_t static_flags(int PT, int PASS) {
 // occupancy with the extra registers: T1 with 16-bit state and 16-bit params, reference-default
 // flags (in one process, bf16-state cfg4 1.653 -> 1.612 ms, fp16 cfg4 1.996 -> 1.904 ms). With
 // 2 sub-units the T2 and TD-CLM 16-bit kernels and T1's other flag words need more registers than
-// 8 waves per SIMD leave, and spill.
+// 8 waves per SIMD leave, and spill. The counting pass of a large launch only reads, 6 to 12 bytes an
+// element, and a block of 1024 elements is mostly its own prologue: with 4096-element units, all their
+// loads in flight at once, the two passes of a 9.5e8-element bf16 step run 3450 -> 3071 us (TD-CLM)
+// and 5249 -> 4972 us (CLM), of a 1.2e8-element f32 step 821 -> 774 us (CLM); 2048-element units 3089,
+// 5060 and 774. Small launches lose (3.5e6 elements 22.1 -> 23.5 us) and keep 1024 or 2048.
 constexpr int unit_subs(int mode, int pt, int st, int pass, uint32_t flags) {
+    if (pass == kCount) return (flags & kFLarge) ? 4 / unit_halves(mode, pt, st) : 1;
     return (mode == LV_BUFFER_T1 && st != LV_DTYPE_F32 && pt != LV_DTYPE_F32 && flags == static_flags(pt, pass)) ? 2 : 1;
 }
 
@@ -99,7 +104,7 @@ constexpr int unit_subs(int mode, int pt, int st, int pass, uint32_t flags) {
 // registers for a second sub-unit's loads out of occupancy (102 SGPRs: 7 waves per SIMD, where
 // the bound keeps 8 and 78 SGPRs): 1.635 against 1.612 ms for bf16-state cfg4.
 constexpr int unit_min_blocks(int mode, int pt, int st, int pass, uint32_t flags) {
-    return unit_subs(mode, pt, st, pass, flags) > 1 ? 8 : 1;
+    return unit_subs(mode, pt, st, pass, flags) > 1 && pass != kCount ? 8 : 1;
 }
 
 // Resident one-wave blocks per CU of a large f32-state launch, 0 where it keeps 256-thread blocks.
@@ -143,26 +148,29 @@ constexpr uint32_t wave_resident(int mode, int pt, bool master, bool table) {
 // in granules of 1280 bytes, and the kernel's own few bytes stay within the last granule.
 constexpr uint32_t wave_lds_bytes(uint32_t resident) { return resident && resident < 32u ? 128u / resident * 1280u - 256u : 0u; }
 
-// Smallest launch (elements of its class) that takes the one-wave kernels of wave_resident. Below it
+// Smallest launch (elements of its class) that takes the kernels' large forms (unit_large). Below it
 // a CU sees each of its waves only a few times and the limit costs what the order gains: at 4e6
 // elements 0.91-1.02x, at 8e6 0.97-1.02x, at 1.6e7 0.99-1.03x, at 3.2e7 1.01-1.05x (CLM f32, T2 bf16).
-constexpr uint64_t kWaveElems = 1ull << 25;
+constexpr uint64_t kLargeElems = 1ull << 25;
 
-// Whether the kernels of this word have a one-wave form (kFWave): the steady pass with f32 state and
-// the reference defaults, with or without a master copy.
-constexpr bool unit_wave(int mode, int pt, int st, int pass, uint32_t flags, bool table) {
-    return st == LV_DTYPE_F32 && pass == kFused && (flags & ~(uint32_t)(kFMaster | kFWave)) == static_flags(pt, pass) &&
+// Whether the kernels of this word have a form for large launches (kFLarge), with the reference
+// defaults: the passes that write the update, with f32 state and with or without a master copy, in
+// one-wave blocks (wave_resident; non-cautious CLM f32 582.9 -> 536.4 us, 1.2e8 elements unfused);
+// the counting pass in larger units (unit_subs).
+constexpr bool unit_large(int mode, int pt, int st, int pass, uint32_t flags, bool table) {
+    if (pass == kCount) return (flags & ~(uint32_t)kFLarge) == static_flags(pt, pass);
+    return st == LV_DTYPE_F32 && (flags & ~(uint32_t)(kFMaster | kFLarge)) == static_flags(pt, pass) &&
            wave_resident(mode, pt, (flags & kFMaster) != 0, table) != 0;
 }
 
 // Threads per block of the unit kernel for this mode, dtypes, pass, flag word (the launch's word;
-// the run-time-flag kernels have 256) and launch kind. The kFWave kernels run one-wave blocks (units
-// of 256 elements), and so do two steady inline steps with f32 state and the reference defaults at
+// the run-time-flag kernels have 256) and launch kind. The kFLarge kernels that write run one-wave
+// blocks (units of 256 elements), and so do two steady inline steps with f32 state and the reference defaults at
 // every size. In one process on the same buffers, against 256-thread blocks:
 // - CLM in f32 (cfg3's kernel): 0.938-0.966x (cfg3, and a 1e9-element bucket);
 // - T2 with bf16 params (the headline's kernel): 0.966x at 1e9 elements, 0.959x at 3.5e9.
 constexpr int unit_threads(int mode, int pt, int st, int pass, uint32_t flags, bool table) {
-    if (flags & kFWave) return 64;
+    if (flags & kFLarge) return pass == kCount ? kThreads : 64;
     const bool one_wave = (mode == LV_BUFFER_DUAL && pt == LV_DTYPE_F32) || (mode == LV_BUFFER_T2 && pt == LV_DTYPE_BF16);
     return (!table && one_wave && st == LV_DTYPE_F32 && pass == kFused && flags == static_flags(pt, pass)) ? 64 : kThreads;
 }
@@ -1618,7 +1626,7 @@ __global__ void __launch_bounds__(unit_threads(MODE, PT, ST, PASS, FL, TABLE), u
     constexpr int TPB = unit_threads(MODE, PT, ST, PASS, FL, TABLE);  // threads per block
     __shared__ BlockSums<TPB> sh;
 
-    const uint32_t flags = (FL & kFDynamic) ? a.flags : (FL & ~(uint32_t)kFWave);
+    const uint32_t flags = (FL & kFDynamic) ? a.flags : (FL & ~(uint32_t)kFLarge);
     const bool radial = kCounting && (flags & kFRadial);  // squared norms summed in this pass
     // Workgroups are dispatched to the XCDs round-robin (block b runs on XCD b mod X). Map them so
     // that each XCD streams one contiguous range of units, or, where the host passes X = 1, block
@@ -1893,15 +1901,18 @@ template <int MODE, int PT, int ST, int PASS>
 KernelFn pick_flags(uint32_t flags, bool table) {
     constexpr uint32_t kStatic = static_flags(PT, PASS);
     constexpr uint32_t kRadial = radial_flags(PT);
-    if constexpr (PASS == kFused && ST == LV_DTYPE_F32) {  // the one-wave kernels of large launches
-        constexpr uint32_t kW = kStatic | kFWave, kWM = kW | kFMaster;
+    if constexpr (PASS == kCount) {
+        constexpr uint32_t kL = kStatic | kFLarge;
+        if (flags == kL) return table ? unit_kernel<MODE, PT, ST, PASS, kL, true> : unit_kernel<MODE, PT, ST, PASS, kL, false>;
+    } else if constexpr (ST == LV_DTYPE_F32) {  // the one-wave kernels of large launches
+        constexpr uint32_t kW = kStatic | kFLarge, kWM = kW | kFMaster;
         if (flags == kW) {
-            if constexpr (unit_wave(MODE, PT, ST, PASS, kW, true))
+            if constexpr (unit_large(MODE, PT, ST, PASS, kW, true))
                 if (table) return unit_kernel<MODE, PT, ST, PASS, kW, true>;
-            if constexpr (unit_wave(MODE, PT, ST, PASS, kW, false))
+            if constexpr (unit_large(MODE, PT, ST, PASS, kW, false))
                 if (!table) return unit_kernel<MODE, PT, ST, PASS, kW, false>;
         }
-        if constexpr (PT != LV_DTYPE_F32 && unit_wave(MODE, PT, ST, PASS, kWM, true))
+        if constexpr (PT != LV_DTYPE_F32 && unit_large(MODE, PT, ST, PASS, kWM, true))
             if (flags == kWM) return table ? unit_kernel<MODE, PT, ST, PASS, kWM, true> : unit_kernel<MODE, PT, ST, PASS, kWM, false>;
     }
     if (table) {
