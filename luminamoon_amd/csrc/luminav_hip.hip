@@ -719,6 +719,15 @@ static uint64_t desc_units(const Desc &D, uint32_t unit_elems) {
     return units_of(D.n - (D.vec ? D.head : 0u), unit_elems);
 }
 
+// The facts about the hyper-parameters that optimistic lanes (lane_update) rely on. They hold for
+// every step: beta1's bias correction lies in [1 - beta1^2, 1] and beta2's in (0, 1], so c1 and c2 are
+// at least their first factors below. `args` has the derived constants.
+static bool lane_facts(const lv_config *cfg, const Args &args) {
+    if (!(args.ranges & kRangeM) || !(args.ranges & kRangeP) || !(cfg->bound_ratio >= 0x1p-20f)) return false;
+    if (cfg->buffer == LV_BUFFER_DUAL) return args.omb1sq * cfg->tau * cfg->eps >= 1.1e-12f;
+    return args.b1sq >= 0x1p-20f && args.omb1sq >= 0x1p-20f && cfg->eps >= 0x1p-40f;
+}
+
 // kLargeElems, or LV_LARGE_ELEMS (so tests can run the kernels of large launches on small ones).
 static uint64_t large_elems() {
     const char *e = std::getenv("LV_LARGE_ELEMS");
@@ -767,7 +776,9 @@ static void fill_args_common(Args &args, const lv_config *cfg, const Item &h, in
     // A counting pass without the radial bound reads neither the rounding, the decay, the bound nor the
     // master options: it takes the kernel of the reference defaults.
     if (h.pass == kCount && bound != LV_BOUND_RADIAL && cfg->cautious && h.gt == h.pt) flags = static_flags(h.pt, kCount);
-    if (elems >= large_elems() && unit_large(cfg->buffer, h.pt, h.st, h.pass, flags, table)) flags |= kFLarge;
+    if (elems >= large_elems() && unit_large(cfg->buffer, h.pt, h.st, h.pass, flags, table) &&
+        (!unit_lanes(cfg->buffer, h.pt, h.st, h.pass, flags | kFLarge) || lane_facts(cfg, args)))
+        flags |= kFLarge;
     args.flags = flags;
 }
 

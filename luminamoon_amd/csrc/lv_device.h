@@ -83,6 +83,25 @@ constexpr uint32_t static_flags(int PT, int PASS) {
            (uint32_t)kFCoordinate | (PT == LV_DTYPE_F16 ? (uint32_t)kFClampV : 0u) | ((uint32_t)PT << 8);
 }
 
+// Whether the whole-unit vector path of this kernel runs optimistic lanes (lane_update): straight-line
+// arithmetic for the common case, one range test per thread at the end, and the general path for a
+// wave that fails it. For the large forms of the steps that their arithmetic bounds: CLM and TD-CLM
+// with 16-bit params, cautious, no master copy. Against the general path, in one process on the same
+// buffers (9.5e8 elements):
+//   CLM  bf16, bf16 state 3224.6 -> 2871.9 us    CLM bf16, f32 state 3467.4 -> 3387.9 us
+//   TD   bf16, bf16 state 2116.7 -> 1990.0       TD  bf16, f32 state 2308.4 -> 2128.1
+//   CLM  f16,  f32 state  4123.3 -> 3826.3       TD  f16,  f32 state 3079.7 -> 2807.7
+// and the same with 5% of the gradients zero for thousands of steps (m and v decayed away there): 3238.4
+// -> 2872.8 and 3726.8 -> 3422.1. T1 and T2 with 16-bit state measured 0.97-0.99x (their general path has
+// one guarded quotient less and no tanh), CLM f16 with 16-bit state 0.79x (it spills).
+constexpr bool unit_lanes(int mode, int pt, int st, int pass, uint32_t flags) {
+    const uint32_t need = (uint32_t)kFLarge | (uint32_t)kFCautious | (uint32_t)kFSR | (uint32_t)kFWeightDecay | (uint32_t)kFCoordinate;
+    return pass != kCount && (flags & (need | (uint32_t)kFRadial | (uint32_t)kFMaster)) == need &&
+           (mode == LV_BUFFER_DUAL || mode == LV_BUFFER_TDCLM) &&
+           (pt == LV_DTYPE_BF16 || (pt == LV_DTYPE_F16 && st == LV_DTYPE_F32));
+}
+constexpr int kLaneGroup = 2;  // elements of a lane whose arithmetic is interleaved
+
 // Sub-units per work unit (each 1024 * unit_halves elements) of the kernel for this mode, dtypes,
 // pass and flag word (the launch's word; the run-time-flag kernels have 1). A block of 2 issues
 // the loads of both sub-units before it computes the first, so the second's memory latency hides
@@ -104,6 +123,7 @@ constexpr int unit_subs(int mode, int pt, int st, int pass, uint32_t flags) {
 // registers for a second sub-unit's loads out of occupancy (102 SGPRs: 7 waves per SIMD, where
 // the bound keeps 8 and 78 SGPRs): 1.635 against 1.612 ms for bf16-state cfg4.
 constexpr int unit_min_blocks(int mode, int pt, int st, int pass, uint32_t flags) {
+    if (unit_lanes(mode, pt, st, pass, flags)) return st != LV_DTYPE_F32 ? 8 : 1;
     return unit_subs(mode, pt, st, pass, flags) > 1 && pass != kCount ? 8 : 1;
 }
 
@@ -135,13 +155,16 @@ constexpr int unit_min_blocks(int mode, int pt, int st, int pass, uint32_t flags
 // More arithmetic per byte needs more waves, more bytes per wave fewer. T1 with 16-bit params and no
 // master moves too few bytes per wave for a limit (table 2152 -> 2071 at 32 per CU, 2163 at 25; its
 // inline launches stay level with 256-thread blocks, 2069). CLM and TD-CLM with 16-bit params and no
-// master are bound by their arithmetic: CLM f16 4143 -> 4167, TD bf16 2336 -> 2331 at 32 per CU.
+// master are bound by their arithmetic, and one-wave blocks alone change nothing there (CLM f16 4143 ->
+// 4167, TD bf16 2336 -> 2331); with optimistic lanes (unit_lanes): CLM bf16 32: 3511.9  25: 3459.5  21:
+// 3387.9, CLM f16 32: 3826.3  25: 3847.3, TD bf16 32: 2125.4  25: 2255.9, TD f16 32: 2802.1  25: 2832.7.
 constexpr uint32_t wave_resident(int mode, int pt, bool master, bool table) {
     if (pt == LV_DTYPE_F32)
         return mode == LV_BUFFER_T2 ? 16u : mode == LV_BUFFER_TDCLM ? 21u : 18u;
     if (master) return mode == LV_BUFFER_TDCLM ? 25u : mode == LV_BUFFER_DUAL ? 21u : mode == LV_BUFFER_T1 ? 18u : 16u;
     if (mode == LV_BUFFER_T2) return pt == LV_DTYPE_BF16 ? 18u : 25u;
-    return mode == LV_BUFFER_T1 && table ? 32u : 0u;
+    if (mode == LV_BUFFER_DUAL && pt == LV_DTYPE_BF16) return 21u;
+    return mode == LV_BUFFER_T1 && !table ? 0u : 32u;
 }
 
 // Dynamic LDS bytes of a one-wave block that leave room for `resident` blocks on a CU: LDS is 160 KB
@@ -159,8 +182,10 @@ constexpr uint64_t kLargeElems = 1ull << 25;
 // the counting pass in larger units (unit_subs).
 constexpr bool unit_large(int mode, int pt, int st, int pass, uint32_t flags, bool table) {
     if (pass == kCount) return (flags & ~(uint32_t)kFLarge) == static_flags(pt, pass);
-    return st == LV_DTYPE_F32 && (flags & ~(uint32_t)(kFMaster | kFLarge)) == static_flags(pt, pass) &&
-           wave_resident(mode, pt, (flags & kFMaster) != 0, table) != 0;
+    if ((flags & ~(uint32_t)(kFMaster | kFLarge)) != static_flags(pt, pass)) return false;
+    const bool arithmetic = (mode == LV_BUFFER_DUAL || mode == LV_BUFFER_TDCLM) && pt != LV_DTYPE_F32 && !(flags & kFMaster);
+    if (st != LV_DTYPE_F32 || arithmetic) return unit_lanes(mode, pt, st, pass, flags | kFLarge);
+    return wave_resident(mode, pt, (flags & kFMaster) != 0, table) != 0;
 }
 
 // Threads per block of the unit kernel for this mode, dtypes, pass, flag word (the launch's word;
@@ -170,7 +195,7 @@ constexpr bool unit_large(int mode, int pt, int st, int pass, uint32_t flags, bo
 // - CLM in f32 (cfg3's kernel): 0.938-0.966x (cfg3, and a 1e9-element bucket);
 // - T2 with bf16 params (the headline's kernel): 0.966x at 1e9 elements, 0.959x at 3.5e9.
 constexpr int unit_threads(int mode, int pt, int st, int pass, uint32_t flags, bool table) {
-    if (flags & kFLarge) return pass == kCount ? kThreads : 64;
+    if (flags & kFLarge) return pass == kCount ? kThreads : st != LV_DTYPE_F32 ? kThreads : 64;
     const bool one_wave = (mode == LV_BUFFER_DUAL && pt == LV_DTYPE_F32) || (mode == LV_BUFFER_T2 && pt == LV_DTYPE_BF16);
     return (!table && one_wave && st == LV_DTYPE_F32 && pass == kFused && flags == static_flags(pt, pass)) ? 64 : kThreads;
 }
@@ -1104,6 +1129,190 @@ __device__ __forceinline__ void count_elem(const Args &a, const StepCoeffs &k, c
     u_eff = (flags & kFCautious) ? u * (active ? 1.0f : 0.0f) : u;
 }
 
+// ------------------------------------------------------------------ optimistic lanes
+
+// Range facts of the elements a thread has updated with lane_update: the largest of the magnitudes
+// that must stay below kLaneMax (hi: NaN if any is NaN; den: NaNs ignored), and the lanes of the wave
+// with a nonzero gradient whose u or v' is below its bound (wave-uniform).
+struct LaneRange {
+    float hi = 0.0f, den = 0.0f;
+    uint64_t low = 0;
+};
+
+// Bounds lane_update's arithmetic relies on. They hold for the values of training runs by many
+// orders of magnitude, dead elements (zero gradients for any number of steps, m and v decayed to
+// subnormals or zero) included: what fails them is broken state and a few exact cancellations.
+constexpr float kLaneMax = 0x1p25f;    // |g|, |g - m'|, |v'|, the bound's b; sigma or the envelope
+constexpr float kLaneMinV = 0x1p-96f;  // v', where g is not zero
+constexpr float kLaneMinU = 0x1p-57f;  // |u|, where g is not zero; and lr |u| cs >= kLaneMinStep
+constexpr float kLaneMinStep = 0x1p-45f;
+
+// The smallest |u| at which the step lr * u * cs is at least kLaneMinStep; infinity (no element with
+// a gradient passes) when lr * cs is 0, negative, above 2^40 or NaN.
+__device__ __forceinline__ float lane_min_u(float lr, float cs) {
+    const float s = lr * cs;
+    const float t = __builtin_fmaxf(kLaneMinU, kLaneMinStep * __builtin_amdgcn_rcpf(s));
+    return (s > 0.0f && s <= 0x1p40f) ? t : __builtin_inff();
+}
+
+// tanh_pade of an x that is not NaN and zero or at least 2^-92 in magnitude: the quotient's
+// numerator is zero or at least 2^-100 and its denominator lies in [2^-8, 2], so div_unscaled is
+// exact up to the sign of a zero.
+__device__ __forceinline__ float tanh_lane(float x_in, const PadeK &c) {
+    const float x = __builtin_amdgcn_fmed3f(x_in, -7.9988117f, c.hi);
+    const float x2 = x * x;
+    float p = __builtin_fmaf(c.p0, x2, 2.000188e-13f);
+    float q = __builtin_fmaf(c.q0, x2, 1.1853471e-4f);
+    p = __builtin_fmaf(p, x2, -8.604672e-11f);
+    q = __builtin_fmaf(q, x2, 2.2684346e-3f);
+    p = __builtin_fmaf(p, x2, 5.122297e-8f);
+    q = __builtin_fmaf(q, x2, 4.8935246e-3f);
+    p = __builtin_fmaf(p, x2, 1.4857224e-5f);
+    p = __builtin_fmaf(p, x2, 6.3726193e-4f);
+    p = __builtin_fmaf(p, x2, 4.8935246e-3f);
+    return div_unscaled(x * p, q);
+}
+
+__device__ __forceinline__ void lane_hi(LaneRange &r, float x) {
+    r.hi = __builtin_elementwise_maximum(r.hi, __builtin_fabsf(x));  // NaN propagates
+}
+
+// One element of an optimistic lane, CLM or TD-CLM: apply_elem's update (cautious, coordinate bound,
+// weight decay, stochastic rounding) without a wave-uniform guard, gathering in `r` what must hold
+// for its result to be apply_elem's. The caller takes the results only if `r` passes in every lane of
+// the wave (lane_ok); the launch has checked lane_facts. cs: the cautious scale; min_u: lane_min_u.
+//
+// Why the result is apply_elem's when r passes. No value in r.hi is NaN, so g, m, v' and p are not.
+// - sanitize and clamp_defect are the identity. CLM: |g|, |g - m'| <= 2^25. TD-CLM: r.den bounds the
+//   envelope, at least (1 - b1^2) |g| and b1^2 |m| with both factors >= 2^-20, so |g|, |m| <= 2^45.
+// - an element with g = 0 is masked: u * g is not above 0 whatever u is (NaN included), its step is 0,
+//   and m', v' do not depend on u. Otherwise:
+// - CLM: v' is in [2^-96, 2^25], so the clamp at 0 is the identity and sqrt_rn_positive is the root,
+//   and sigma >= c2 >= 1e-12, so its floor is the identity.
+// - u's quotient: the denominator lies in [2^-40, 2^25]. Were |clm| below 2^-100, u would come out
+//   below 2^-57 and fail min_u, so div_unscaled is exact; |u| <= 1 + 2^-20.
+// - the bound: active elements have 2^-46 <= |step| <= 2^41 (min_u); masked ones a zero of either sign,
+//   which weight decay makes irrelevant (div_bound). b = ratio sqrt(p^2 + 1e-4) lies in [2^-27, 2^25]
+//   (ratio >= 2^-20), so step / b is at least 2^-71 and at most 2^68 and b tanh(step / b) at least
+//   2^-47.
+// - the fp16 safety bound after it: |p| <= 2^45, so its b lies in [1.5e-4, 2^39] and its quotients in
+//   div_unscaled's domain.
+// - the roundings: |m'| <= 2^46, |v'| <= 2^25 and |p'| < 2^86 (kRangeP) need no range test.
+template <int MODE, int PT, int ST, int TALLY>
+__device__ __forceinline__ void lane_update(const Args &a, const StepCoeffs &k, const LaneK &lk, uint32_t flags,
+                                            const HashIn &z, float cs, float min_u, float p_init, float g, float &m_io,
+                                            float &v_io, float &p_out, uint32_t &cnt, LaneRange &r) {
+    constexpr bool kDual = MODE == LV_BUFFER_DUAL;
+    static_assert(kDual || MODE == LV_BUFFER_TDCLM, "CLM and TD-CLM");
+    const float m = m_io;
+    const float og = a.omb1 * g;
+    const float m_new = __builtin_fmaf(a.b1, m, og);
+    const uint64_t has_g = __builtin_amdgcn_ballot_w64(g != 0.0f);
+    float u, v_new = 0.0f;
+    if constexpr (kDual) {
+        const float clm = __builtin_fmaf(a.b1, m_new, og);
+        const float diff = g - m_new;
+        v_new = __builtin_fmaf(a.b2, v_io, a.omb2 * (diff * diff));
+        if (flags & kFClampV) v_new = __builtin_fminf(v_new, 65000.0f);
+        const float sigma = __builtin_fmaf(sqrt_rn_positive(v_new), k.c1, k.c2);
+        lane_hi(r, g);
+        lane_hi(r, diff);
+        lane_hi(r, v_new);
+        r.den = __builtin_fmaxf(r.den, sigma);  // NaN where v' is 0: an element with no gradient, or r.low
+        r.low |= has_g & __builtin_amdgcn_ballot_w64(v_new < kLaneMinV);
+        u = tanh_lane(div_unscaled(clm, sigma), lk.pade);
+    } else {
+        const float clm = __builtin_fmaf(a.b1sq, m, a.omb1sq * g);
+        const float diff = g - m;
+        const float env = fma_abs(a.lam, diff, __builtin_fmaf(a.omb1sq, fabsf(g), __builtin_fmaf(a.b1sq, fabsf(m), lk.eps)));
+        lane_hi(r, env);
+        u = div_unscaled(clm, env);
+    }
+    r.low |= has_g & __builtin_amdgcn_ballot_w64(fabsf(u) < min_u);
+    const bool active = (u * g) > 0.0f;
+    tally<TALLY>(cnt, active);
+    m_io = quantize_known<ST>(m_new, z.m, true, true);
+    if constexpr (kDual) v_io = quantize_known<ST>(v_new, z.v, true, true);
+    // (u * mask) * cs: selected before the scale, so that a masked element's u need not be a number
+    float step = a.lr * ((active ? u : 0.0f) * cs);
+    const float b = a.ratio * sqrt_rn_positive(__builtin_fmaf(p_init, p_init, 1.0e-4f));
+    lane_hi(r, b);
+    step = b * tanh_lane(div_unscaled(step, b), lk.pade);
+    if constexpr (PT == LV_DTYPE_F16) {
+        const float bs = __builtin_fmaxf(fabsf(p_init) * 0.01f, 1.5e-4f);
+        step = bs * tanh_lane(div_unscaled(step, bs), lk.pade);
+    }
+    const float p_upd = __builtin_fmaf(a.neg_lr_wd, p_init, p_init) - step;
+    if constexpr (PT == LV_DTYPE_F16) p_out = sr_fp16_val(p_upd, z.p);
+    else p_out = quantize_known<PT>(p_upd, z.p, true, true);
+}
+
+// Every lane of the wave passes its range test, and the scale is one lane_min_u has a bound for.
+__device__ __forceinline__ bool lane_ok(const LaneRange &r, float min_u) {
+    return wave_all((r.hi <= kLaneMax) & (r.den <= kLaneMax) & (min_u < __builtin_inff())) && r.low == 0;
+}
+
+// Element j of a raw lane (decode_raw's j-th output).
+template <int DT>
+__device__ __forceinline__ float lane_get(const Raw8 &r, int j) {
+    if constexpr (DT == LV_DTYPE_F32) return bits_f(j < 4 ? r.a[j] : r.b[j - 4]);
+    else if constexpr (DT == LV_DTYPE_BF16) return bits_f((j & 1) ? r.a[j / 2] & 0xFFFF0000u : r.a[j / 2] << 16);
+    else return f16_to_f32((j & 1) ? r.a[j / 2] >> 16 : r.a[j / 2] & 0xFFFFu);
+}
+
+// Holds back the arithmetic of elements [j, j + kLaneGroup) of a raw stream until the results before them are
+// kept (lane_keep; the volatile statements stay in order).
+template <int DT>
+__device__ __forceinline__ void lane_hold(Raw8 &r, int j) {
+#pragma unroll
+    for (int i = j; i < j + kLaneGroup; i += DT == LV_DTYPE_F32 ? 1 : 2) {
+        const int w = DT == LV_DTYPE_F32 ? i & 3 : i / 2;
+        if (DT != LV_DTYPE_F32 || i < 4) {
+            uint32_t t = r.a[w];
+            asm volatile("" : "+v"(t));
+            r.a[w] = t;
+        } else {
+            uint32_t t = r.b[w];
+            asm volatile("" : "+v"(t));
+            r.b[w] = t;
+        }
+    }
+}
+
+// Keeps the lane's j-th result where it is computed: the results are only stored behind the lane's
+// range test, and the compiler would otherwise sink every element's roundings and hashes there and
+// carry their f32 inputs (and spill). 16-bit results are packed as soon as a pair is complete, two to
+// a word in x[j / 2] (store_lane).
+template <int DT>
+__device__ __forceinline__ void lane_keep(float x[8], int j) {
+    if constexpr (DT == LV_DTYPE_F32) {
+        asm volatile("" : "+v"(x[j]));
+    } else if (j & 1) {
+        uint32_t w;
+        if constexpr (DT == LV_DTYPE_BF16) w = __builtin_amdgcn_perm(f_bits(x[j]), f_bits(x[j - 1]), 0x07060302u);
+        else w = pack_f16_rtz(x[j - 1], x[j]);
+        asm volatile("" : "+v"(w));
+        x[j / 2] = bits_f(w);
+    }
+}
+
+// store_raw of a lane's 4 * H results kept by lane_keep.
+template <int DT, int H, uint32_t HS>
+__device__ __forceinline__ void store_lane(void *base, uint64_t h0, const float x[8]) {
+    if constexpr (DT == LV_DTYPE_F32) {
+        store_raw<DT, H, HS>(base, h0, x);
+    } else {
+        LV_GLOBAL uint16_t *h = (LV_GLOBAL uint16_t *)base;
+        if constexpr (H == 2 && HS == 4) {
+            __builtin_nontemporal_store(f32x4{x[0], x[1], x[2], x[3]}, (LV_GLOBAL f32x4 *)(h + h0));
+        } else {
+            __builtin_nontemporal_store(u32x2{f_bits(x[0]), f_bits(x[1])}, (LV_GLOBAL u32x2 *)(h + h0));
+            if constexpr (H == 2)
+                __builtin_nontemporal_store(u32x2{f_bits(x[2]), f_bits(x[3])}, (LV_GLOBAL u32x2 *)(h + h0 + HS));
+        }
+    }
+}
+
 // ------------------------------------------------------------------ scratch finalisation
 
 // Last block of tensor t: dual.rs:255-259 + math.rs:188-239 (fused), dual.rs:330-351 +
@@ -1328,11 +1537,11 @@ __device__ __forceinline__ Inflight issue_at(const Desc &D, uint32_t flags, bool
 // operand. eps is read by T1, T2 and TD-CLM, the tanh constants by CLM and TD-CLM (tanh_pade).
 // CLM with 16-bit state keeps the tanh constants as they are: there the extra VGPRs would cost
 // some of its kernels a wave of occupancy (T2's eps costs none of its kernels one).
-template <int MODE, int H>
+template <int MODE, int H, bool LANES = false>
 __device__ __forceinline__ LaneK lane_consts(const Args &a) {
     LaneK lk{a.eps, kPade};
     if constexpr (MODE == LV_BUFFER_T1 || MODE == LV_BUFFER_TDCLM || MODE == LV_BUFFER_T2) lk.eps = in_vgpr(a.eps);
-    if constexpr (MODE == LV_BUFFER_TDCLM || (MODE == LV_BUFFER_DUAL && H == 1))
+    if constexpr (MODE == LV_BUFFER_TDCLM || (MODE == LV_BUFFER_DUAL && (H == 1 || LANES)))
         lk.pade = PadeK{in_vgpr(kPade.hi), in_vgpr(kPade.p0), in_vgpr(kPade.q0)};
     return lk;
 }
@@ -1340,7 +1549,7 @@ __device__ __forceinline__ LaneK lane_consts(const Args &a) {
 // Update (or count) the 4 * H elements loaded by issue_at(e0) and store them. BALLOT: every lane
 // of the wave is here, and cnt accumulates the wave's count (the same in every lane) from ballots;
 // otherwise cnt accumulates the lane's own count.
-template <int MODE, int PT, int ST, int PASS, int H, bool BALLOT, uint32_t HS = 4>
+template <int MODE, int PT, int ST, int PASS, int H, bool BALLOT, uint32_t HS = 4, bool LANES = false>
 __device__ __forceinline__ void process_at(const Args &a, const Desc &D, const View &tv, uint32_t flags, bool radial,
                                            const Inflight &cur, uint64_t e0, uint32_t &cnt, double &su, double &sp) {
     constexpr bool kDual = (MODE == LV_BUFFER_DUAL || MODE == LV_BUFFER_T2);
@@ -1348,7 +1557,48 @@ __device__ __forceinline__ void process_at(const Args &a, const Desc &D, const V
     constexpr int kTally = !kCounting ? kTallyNone : (BALLOT ? kTallyWave : kTallyLane);
     const int gdt = (int)((flags >> 8) & 3u);
     const bool master = flags & kFMaster;
-    const LaneK lk = lane_consts<MODE, H>(a);
+    const LaneK lk = lane_consts<MODE, H, LANES>(a);
+    if constexpr (LANES) {
+        // Optimistic lanes; a wave that fails the range test loads its elements again and takes the
+        // general path, one group of 4 at a time.
+        float m[8], v[8], pout[8];
+        const HashIn zb = hash_in(tv.sd, (uint32_t)e0 + tv.ibase);
+        const float cs = in_vgpr(tv.cs), min_u = lane_min_u(a.lr, tv.cs);
+        LaneRange r;
+        uint32_t c = 0;
+        Inflight x = cur;
+#pragma unroll
+        for (int j = 0; j < 4 * H; j++) {
+            if (j % kLaneGroup == 0) {
+                lane_hold<PT>(x.g, j);
+                lane_hold<ST>(x.m, j);
+                if constexpr (kDual) lane_hold<ST>(x.v, j);
+                lane_hold<PT>(x.p, j);
+            }
+            const uint32_t off = j < 4 ? (uint32_t)j : HS + (uint32_t)(j - 4);
+            m[j] = lane_get<ST>(x.m, j);
+            v[j] = kDual ? lane_get<ST>(x.v, j) : 0.0f;
+            lane_update<MODE, PT, ST, kTally>(a, tv.k, lk, flags, {zb.m + off, zb.p + off, zb.v + off}, cs, min_u,
+                                              lane_get<PT>(x.p, j), lane_get<PT>(x.g, j), m[j], v[j], pout[j], c, r);
+            lane_keep<PT>(pout, j);
+            lane_keep<ST>(m, j);
+            if constexpr (kDual) lane_keep<ST>(v, j);
+        }
+        if (__builtin_expect(lane_ok(r, min_u), 1)) {
+            cnt += c;
+            store_lane<PT, H, HS>(D.p, e0, pout);
+            store_lane<ST, H, HS>(D.m, e0, m);
+            if constexpr (kDual) store_lane<ST, H, HS>(D.v, e0, v);
+            return;
+        }
+#pragma unroll 1
+        for (int h = 0; h < H; h++) {
+            const uint64_t e = e0 + (uint64_t)h * HS;
+            const Inflight f = issue_at<MODE, PT, ST, PASS, 1>(D, flags, radial, e);
+            process_at<MODE, PT, ST, PASS, 1, BALLOT>(a, D, tv, flags, radial, f, e, cnt, su, sp);
+        }
+        return;
+    }
     float g[8], m[8], v[8];
     decode_raw_dyn<H>(gdt, cur.g, g);
     decode_raw<ST, H>(cur.m, m);
@@ -1564,8 +1814,8 @@ __device__ __forceinline__ void report_count(const Args &a, const Desc &D, const
 // load_raw): 4, so that the thread's 8 elements are consecutive, unless the launch may move an
 // f32 stream beside its 16-bit ones (a master copy, f32 grads, or a flag word known only at run
 // time), then 1024.
-constexpr uint32_t lane_split(int H, uint32_t FL) {
-    return (H == 2 && ((FL & kFDynamic) || (FL & kFMaster) || ((FL >> 8) & 3u) == LV_DTYPE_F32)) ? kHalf : 4u;
+constexpr uint32_t lane_split(int H, uint32_t FL, uint32_t TPB) {
+    return (H == 2 && ((FL & kFDynamic) || (FL & kFMaster) || ((FL >> 8) & 3u) == LV_DTYPE_F32)) ? 4u * TPB : 4u;
 }
 
 // One sub-unit [ub, ub + 1024 * H) of a block that does not take the whole-unit vector path: the
@@ -1661,9 +1911,8 @@ __global__ void __launch_bounds__(unit_threads(MODE, PT, ST, PASS, FL, TABLE), u
     double su = 0.0, sp = 0.0;  // radial: sum u_eff^2, sum p^2
     constexpr int H = unit_halves(MODE, PT, ST);
     constexpr int S = unit_subs(MODE, PT, ST, PASS, FL);
-    constexpr uint32_t HS = lane_split(H, FL);
-    static_assert(H == 1 || TPB == kThreads, "16-bit state splits its lanes at 1024 elements");
-    constexpr uint64_t kSub = 4ull * TPB * H;  // elements per sub-unit
+    constexpr uint32_t HS = lane_split(H, FL, TPB);
+        constexpr uint64_t kSub = 4ull * TPB * H;  // elements per sub-unit
     constexpr uint64_t kUnit = kSub * S;
     // units start at the tensor's first 16-byte aligned element (tv.head > 0: an unaligned view)
     const uint64_t ubase = (uint64_t)(unit - tv.t_begin) * kUnit + tv.head;
@@ -1686,6 +1935,7 @@ __global__ void __launch_bounds__(unit_threads(MODE, PT, ST, PASS, FL, TABLE), u
     const bool vec = fast && ubase + kUnit <= tv.n;
     const uint64_t e0 = ubase + (uint64_t)threadIdx.x * (HS == 4 ? 4u * H : 4u);  // the first group
     if (vec) {
+        constexpr bool kLanes = unit_lanes(MODE, PT, ST, PASS, FL);
         Inflight f[S];
 #pragma unroll
         for (int sub = 0; sub < S; sub++)
@@ -1705,7 +1955,7 @@ __global__ void __launch_bounds__(unit_threads(MODE, PT, ST, PASS, FL, TABLE), u
         __builtin_amdgcn_s_setprio(S == 1 ? 1 : 0);
 #pragma unroll
         for (int sub = 0; sub < S; sub++)
-            process_at<MODE, PT, ST, PASS, H, true, HS>(a, D, tv, flags, radial, f[sub], e0 + (uint64_t)sub * kSub, cnt,
+            process_at<MODE, PT, ST, PASS, H, true, HS, kLanes>(a, D, tv, flags, radial, f[sub], e0 + (uint64_t)sub * kSub, cnt,
                                                        su, sp);
     } else {
         if constexpr (!TABLE) {
@@ -1904,7 +2154,7 @@ KernelFn pick_flags(uint32_t flags, bool table) {
     if constexpr (PASS == kCount) {
         constexpr uint32_t kL = kStatic | kFLarge;
         if (flags == kL) return table ? unit_kernel<MODE, PT, ST, PASS, kL, true> : unit_kernel<MODE, PT, ST, PASS, kL, false>;
-    } else if constexpr (ST == LV_DTYPE_F32) {  // the one-wave kernels of large launches
+    } else {  // the kernels of large launches
         constexpr uint32_t kW = kStatic | kFLarge, kWM = kW | kFMaster;
         if (flags == kW) {
             if constexpr (unit_large(MODE, PT, ST, PASS, kW, true))

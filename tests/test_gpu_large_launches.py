@@ -9,6 +9,7 @@ import pytest
 import torch
 
 from tests.parity_util import TensorSet, group_dict, oracle_config
+from tests.test_gpu_special_values import GRAD_SPECIALS, M_SPECIALS, P_SPECIALS, V_SPECIALS, _assert_same, _inject
 
 pytestmark = pytest.mark.gpu
 
@@ -73,3 +74,71 @@ def test_two_pass_large_launches_match_oracle(buffer, pdt, sdt, extra, count, mo
         torch.cuda.synchronize()
         host.assert_equal(dev, f"step {step}")
     assert all(int(torch.count_nonzero(ws)) == 0 for ws in stepper.workspace._bufs.values())
+
+
+# Waves whose elements leave optimistic lanes' ranges: the kernels compute them again on the general path.
+def _exact_cancellation(host, grads):
+    for m, g in zip(host.m, grads):  # m' or the direction near or at zero beside ordinary elements
+        m[::97] = (g[::97].float() * -(1.0 - 0.81) / 0.81).to(m.dtype)
+
+
+def _dead(host, grads):
+    for i, g in enumerate(grads):  # zero gradients, m and v decayed to subnormals or zero
+        g[::3] = 0.0
+        host.m[i][::3] = 1e-44
+        host.m[i][::6] = 0.0
+        if host.v[i] is not None:
+            host.v[i][::3] = 1e-41
+            host.v[i][::9] = 0.0
+
+
+def _specials(host, grads):
+    for i, g in enumerate(grads):
+        pos = [k for k in (3, 700, 1029, 2050, 3000, 4097) if k < g.numel()]
+        _inject(g, pos, GRAD_SPECIALS, i)
+        _inject(host.m[i], [p + 1 for p in pos if p + 1 < g.numel()], M_SPECIALS, i)
+        _inject(host.p[i], [p + 2 for p in pos if p + 2 < g.numel()], P_SPECIALS, i)
+        if host.v[i] is not None:
+            _inject(host.v[i], [p + 3 for p in pos if p + 3 < g.numel()], V_SPECIALS, i)
+
+
+def _scales(host, grads):
+    for i, s in enumerate(host.sc):
+        s[3] = [0.0, float("nan"), float("inf"), -1.3, 1e30, 1.3][i % 6]
+    grads[1].zero_()
+
+
+@pytest.mark.parametrize("inputs", [_exact_cancellation, _dead, _specials, _scales], ids=lambda f: f.__name__[1:])
+@pytest.mark.parametrize("buffer,pdt,sdt", [
+    (2, "bf16", "bf16"), (2, "bf16", "f32"), (2, "f16", "f32"), (1, "bf16", "bf16"), (1, "bf16", "f32"), (1, "f16", "f32"),
+])
+def test_optimistic_lanes_match_oracle(buffer, pdt, sdt, inputs, monkeypatch):
+    if not torch.cuda.is_available():
+        pytest.skip("needs a ROCm GPU")
+    from luminamoon_amd.optimizer import hip_backend
+    from oracle import oracle as O
+
+    monkeypatch.setenv("LV_LARGE_ELEMS", "1")
+    for extra in ({}, {"bound_ratio": 1e-7}, {"eps": 1e-13}, {"betas": (0.0, 0.999)}, {"lr": 0.0}, {"lr": 1e-9}):
+        group = group_dict(buffer=buffer, state_precision="param" if sdt != "f32" else "fp32", **{"lr": 1e-3, **extra})
+        cfg = oracle_config(O, group)
+        host = TensorSet([4096 + 37, 2048, 1000, 6144, 70_001, 512], pdt, pdt, sdt, buffer == 2, False, 79, m_scale=3e-4)
+        for v in host.v:
+            if v is not None:
+                v.copy_((v.float() ** 2).to(v.dtype))
+        # one step for fp16: a NaN's sign, which IEEE 754 leaves open, becomes the sign of a 65504
+        steps = (2,) if pdt == "f16" else (2, 3)
+        grads = [host.grads(s, 79) for s in steps]
+        inputs(host, grads[0])
+        dev = host.to("cuda")
+        stepper = hip_backend.HipStepper()
+        print(f"[case] lanes {buffer} {pdt}/{sdt} {inputs.__name__} {extra}", flush=True)
+        for step, g in zip(steps, grads):
+            host.oracle_step(O, cfg, g, step, threads=4)
+            dev.hip_step(stepper, group, [x.cuda() for x in g], step)
+            torch.cuda.synchronize()
+            for i in range(len(host.sizes)):
+                for name in ("p", "m", "v", "sc"):
+                    a, b = getattr(host, name)[i], getattr(dev, name)[i]
+                    if a is not None:
+                        _assert_same(a, b, f"{extra} step {step} {name}[{i}]")
