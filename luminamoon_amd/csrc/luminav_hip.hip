@@ -352,8 +352,9 @@ static void call_needs(const lv_config *cfg, const lv_tensor *T, int count, uint
 // left (the steady step of a many-tensor group) records no event: the slot is marked `pending`,
 // and whoever next needs the event records it on the null stream first, which covers every
 // reader enqueued there (the null stream cannot be destroyed, so that record is always valid).
-// That spares one hipEventRecord of host time per step.
-constexpr int kRingSlots = 4;
+// That spares one hipEventRecord of host time per step. A step takes a table per class and, in a large
+// two-pass launch, per pass: eight hold four such classes.
+constexpr int kRingSlots = 8;
 
 struct TableSlot {
     TDesc *dev = nullptr;
@@ -728,12 +729,6 @@ static bool lane_facts(const lv_config *cfg, const Args &args) {
     return args.b1sq >= 0x1p-20f && args.omb1sq >= 0x1p-20f && cfg->eps >= 0x1p-40f;
 }
 
-// kLargeElems, or LV_LARGE_ELEMS (so tests can run the kernels of large launches on small ones).
-static uint64_t large_elems() {
-    const char *e = std::getenv("LV_LARGE_ELEMS");
-    return e ? std::strtoull(e, nullptr, 10) : kLargeElems;
-}
-
 // `elems`: the elements of the launch's class.
 static void fill_args_common(Args &args, const lv_config *cfg, const Item &h, int bound, uint64_t elems, bool table) {
     std::memset(&args, 0, sizeof args);
@@ -776,7 +771,7 @@ static void fill_args_common(Args &args, const lv_config *cfg, const Item &h, in
     // A counting pass without the radial bound reads neither the rounding, the decay, the bound nor the
     // master options: it takes the kernel of the reference defaults.
     if (h.pass == kCount && bound != LV_BOUND_RADIAL && cfg->cautious && h.gt == h.pt) flags = static_flags(h.pt, kCount);
-    if (elems >= large_elems() && unit_large(cfg->buffer, h.pt, h.st, h.pass, flags, table) &&
+    if (elems >= kLargeElems && unit_large(cfg->buffer, h.pt, h.st, h.pass, flags, table) &&
         (!unit_lanes(cfg->buffer, h.pt, h.st, h.pass, flags | kFLarge) || lane_facts(cfg, args)))
         flags |= kFLarge;
     args.flags = flags;

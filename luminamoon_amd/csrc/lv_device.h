@@ -1912,7 +1912,7 @@ __global__ void __launch_bounds__(unit_threads(MODE, PT, ST, PASS, FL, TABLE), u
     constexpr int H = unit_halves(MODE, PT, ST);
     constexpr int S = unit_subs(MODE, PT, ST, PASS, FL);
     constexpr uint32_t HS = lane_split(H, FL, TPB);
-        constexpr uint64_t kSub = 4ull * TPB * H;  // elements per sub-unit
+    constexpr uint64_t kSub = 4ull * TPB * H;  // elements per sub-unit
     constexpr uint64_t kUnit = kSub * S;
     // units start at the tensor's first 16-byte aligned element (tv.head > 0: an unaligned view)
     const uint64_t ubase = (uint64_t)(unit - tv.t_begin) * kUnit + tv.head;

@@ -1,6 +1,6 @@
-"""The kernels of large launches (kFLarge), run on small launches by lowering their size threshold
-(LV_LARGE_ELEMS): the one-wave kernels with f32 state, the counting pass in 4096-element units with any
-state. Sizes around the 256-element unit, the 1024 elements behind a count slot, the 64 slots and the
+"""The kernels of large launches (kFLarge): the one-wave kernels with f32 state, the counting pass in
+4096-element units with any state, optimistic lanes. A zero tensor of 2^25 elements on the device alone
+makes the launch large; the small tensors before it are compared. Sizes around the 256-element unit, the 1024 elements behind a count slot, the 64 slots and the
 4096-element unit, table and inline launches, with and without a master copy, against the oracle
 bit for bit (the arithmetic is the other kernels', so any difference is an addressing or count error)."""
 from __future__ import annotations
@@ -14,6 +14,21 @@ from tests.test_gpu_special_values import GRAD_SPECIALS, M_SPECIALS, P_SPECIALS,
 pytestmark = pytest.mark.gpu
 
 EDGES = [1, 3, 255, 256, 257, 511, 1023, 1024, 1025, 4095, 4097, 8192 + 2049, 64 * 256, 64 * 1024 - 1, 64 * 1024 + 1, 70_001]
+LARGE = 1 << 25  # kLargeElems
+
+
+def _large(host):
+    """The device copy of `host` with a last tensor of LARGE zeros, and that tensor's gradient."""
+    dev = host.to("cuda")
+    dev.sizes = host.sizes + [LARGE]
+
+    def zeros(like):
+        return None if like[0] is None else torch.zeros(LARGE, dtype=like[0].dtype, device="cuda")
+
+    for xs in (dev.p, dev.m, dev.v, dev.mp):
+        xs.append(zeros(xs))
+    dev.sc.append(torch.tensor([0, 0, 0, 1, 1, 0], dtype=torch.float32, device="cuda"))
+    return dev, torch.zeros(LARGE, dtype=host.gdt, device="cuda")
 
 
 @pytest.mark.parametrize("count", [len(EDGES), 60], ids=["inline", "table"])
@@ -23,24 +38,23 @@ EDGES = [1, 3, 255, 256, 257, 511, 1023, 1024, 1025, 4095, 4097, 8192 + 2049, 64
     (2, "bf16", "full"), (2, "f16", "semi"), ("T2", "bf16", "full"), ("T2", "f16", "full"),
     (1, "bf16", "full"), (1, "f16", "full"), ("T1", "bf16", "semi"), ("T1", "f16", "full"),
 ])
-def test_one_wave_launches_match_oracle(buffer, pdt, master, count, monkeypatch):
+def test_one_wave_launches_match_oracle(buffer, pdt, master, count):
     if not torch.cuda.is_available():
         pytest.skip("needs a ROCm GPU")
     from luminamoon_amd.optimizer import hip_backend
     from oracle import oracle as O
 
-    monkeypatch.setenv("LV_LARGE_ELEMS", "1")
     group = group_dict(buffer=buffer, lr=1e-3, master_weights=master)
     cfg = oracle_config(O, group)
     sizes = [EDGES[i % len(EDGES)] for i in range(count)]
     host = TensorSet(sizes, pdt, pdt, "f32", buffer in (2, "T2"), master != "none", 77)
-    dev = host.to("cuda")
+    dev, fill = _large(host)
     stepper = hip_backend.HipStepper()
     print(f"[case] one-wave {buffer} {pdt} master={master} tensors={count}", flush=True)
     for step in (1, 2, 3):
         grads = host.grads(step, 77)
         host.oracle_step(O, cfg, grads, step, threads=4)
-        dev.hip_step(stepper, group, [g.cuda() for g in grads], step)
+        dev.hip_step(stepper, group, [g.cuda() for g in grads] + [fill], step)
         torch.cuda.synchronize()
         host.assert_equal(dev, f"step {step}")
     assert all(int(torch.count_nonzero(ws)) == 0 for ws in stepper.workspace._bufs.values())
@@ -52,25 +66,24 @@ def test_one_wave_launches_match_oracle(buffer, pdt, master, count, monkeypatch)
     (2, "bf16", "bf16", {"state_precision": "param"}), (2, "bf16", "f32", {"master_weights": "full"}),
     ("T2", "f16", "f32", {"stochastic_rounding": False, "weight_decay": 0.0}), (1, "f32", "f32", {"bound": False}),
 ])
-def test_two_pass_large_launches_match_oracle(buffer, pdt, sdt, extra, count, monkeypatch):
+def test_two_pass_large_launches_match_oracle(buffer, pdt, sdt, extra, count):
     """Counting and applying passes take units of their own kernels' sizes."""
     if not torch.cuda.is_available():
         pytest.skip("needs a ROCm GPU")
     from luminamoon_amd.optimizer import hip_backend
     from oracle import oracle as O
 
-    monkeypatch.setenv("LV_LARGE_ELEMS", "1")
     group = group_dict(buffer=buffer, lr=1e-3, fused_single_pass=False, **extra)
     cfg = oracle_config(O, group)
     sizes = [EDGES[i % len(EDGES)] for i in range(count)]
     host = TensorSet(sizes, pdt, pdt, sdt, buffer in (2, "T2"), "master_weights" in extra, 78)
-    dev = host.to("cuda")
+    dev, fill = _large(host)
     stepper = hip_backend.HipStepper()
     print(f"[case] two-pass {buffer} {pdt}/{sdt} {extra} tensors={count}", flush=True)
     for step in (1, 2):
         grads = host.grads(step, 78)
         host.oracle_step(O, cfg, grads, step, threads=4)
-        dev.hip_step(stepper, group, [g.cuda() for g in grads], step)
+        dev.hip_step(stepper, group, [g.cuda() for g in grads] + [fill], step)
         torch.cuda.synchronize()
         host.assert_equal(dev, f"step {step}")
     assert all(int(torch.count_nonzero(ws)) == 0 for ws in stepper.workspace._bufs.values())
@@ -112,13 +125,12 @@ def _scales(host, grads):
 @pytest.mark.parametrize("buffer,pdt,sdt", [
     (2, "bf16", "bf16"), (2, "bf16", "f32"), (2, "f16", "f32"), (1, "bf16", "bf16"), (1, "bf16", "f32"), (1, "f16", "f32"),
 ])
-def test_optimistic_lanes_match_oracle(buffer, pdt, sdt, inputs, monkeypatch):
+def test_optimistic_lanes_match_oracle(buffer, pdt, sdt, inputs):
     if not torch.cuda.is_available():
         pytest.skip("needs a ROCm GPU")
     from luminamoon_amd.optimizer import hip_backend
     from oracle import oracle as O
 
-    monkeypatch.setenv("LV_LARGE_ELEMS", "1")
     for extra in ({}, {"bound_ratio": 1e-7}, {"eps": 1e-13}, {"betas": (0.0, 0.999)}, {"lr": 0.0}, {"lr": 1e-9}):
         group = group_dict(buffer=buffer, state_precision="param" if sdt != "f32" else "fp32", **{"lr": 1e-3, **extra})
         cfg = oracle_config(O, group)
@@ -130,12 +142,12 @@ def test_optimistic_lanes_match_oracle(buffer, pdt, sdt, inputs, monkeypatch):
         steps = (2,) if pdt == "f16" else (2, 3)
         grads = [host.grads(s, 79) for s in steps]
         inputs(host, grads[0])
-        dev = host.to("cuda")
+        dev, fill = _large(host)
         stepper = hip_backend.HipStepper()
         print(f"[case] lanes {buffer} {pdt}/{sdt} {inputs.__name__} {extra}", flush=True)
         for step, g in zip(steps, grads):
             host.oracle_step(O, cfg, g, step, threads=4)
-            dev.hip_step(stepper, group, [x.cuda() for x in g], step)
+            dev.hip_step(stepper, group, [x.cuda() for x in g] + [fill], step)
             torch.cuda.synchronize()
             for i in range(len(host.sizes)):
                 for name in ("p", "m", "v", "sc"):
