@@ -112,6 +112,10 @@ static int validate_config(const lv_config *c) {
 
 // f32-state unit launches of at most this many blocks map block b to unit b (launch()).
 constexpr uint32_t kIdentityMapUnits = 1u << 21;
+// Largest identity-mapped f32 radial launch of a one-buffer mode, in units (launch()).
+constexpr uint32_t kRadialOneBufferUnits = 1u << 17;
+// f32 radial launches of at least this many (1024-element) units hold fewer blocks per CU (launch()).
+constexpr uint32_t kRadialLimitUnits = 1u << 14;
 
 // XCDs of the current device (hipDeviceAttributeNumberOfXccs; 1 if unknown).
 static uint32_t device_xcds() {
@@ -583,7 +587,16 @@ static int launch(Args &args, int mode, int pt, int st, int pass, hipStream_t st
     // at 1e9 and 3.5e9 elements and 2% faster at 6.7e9; 16-bit-state launches ran level to 4.6%
     // slower. Results are the same either way: units are independent and the count is exact in
     // any order.
-    const bool identity_map = st == LV_DTYPE_F32 && !radial &&
+    // The fused radial step in f32 with the reference defaults (1.2e8 elements unfused): T2 624.9 ->
+    // 604.5 us, CLM (a bucket) 598.5 -> 566.0, TD-CLM 443.4 -> 426.7, T1 444.3 -> 438.9. Above 2^17
+    // units TD-CLM and T1 measured level to 3% slower (2.5e8 elements 792.4 -> 815.0 and 820.5 ->
+    // 815.3) and keep the other mapping. The other radial launches measured mixed and keep it too:
+    // bf16 params CLM 3444.7 -> 3368.2, T2 3572.6 -> 3596.8, TD-CLM 2307.4 -> 2346.1; run-time flags
+    // CLM f32 628.6 -> 638.5; two passes CLM f32 915.7 -> 950.3.
+    const bool radial_f32 = radial && pass == kFused && pt == LV_DTYPE_F32 && st == LV_DTYPE_F32 &&
+                            args.flags == radial_flags(LV_DTYPE_F32) &&
+                            (mode == LV_BUFFER_DUAL || mode == LV_BUFFER_T2 || args.total_units <= kRadialOneBufferUnits);
+    const bool identity_map = st == LV_DTYPE_F32 && (!radial || radial_f32) &&
                               (unit_threads(mode, pt, st, pass, args.flags, table) < kThreads ||
                                args.total_units <= kIdentityMapUnits);
     args.xcds = identity_map ? 1u : device_xcds();
@@ -605,8 +618,17 @@ static int launch(Args &args, int mode, int pt, int st, int pass, hipStream_t st
     if (max_grid == 0) return fail(LV_STATUS_INVALID_CONFIG, "no radial unit records in the workspace");
     KernelFn fold = radial ? pick_fold(mode, pass) : nullptr;
     const uint32_t threads = unit_threads(mode, pt, st, pass, args.flags, table);
-    // one-wave blocks of a large launch: as many per CU as HBM streams best with (wave_resident)
-    const uint32_t lds = threads < kThreads && (args.flags & kFLarge) ? wave_lds_bytes(wave_resident(mode, pt, (args.flags & kFMaster) != 0, table)) : 0u;
+    // One-wave blocks of a large launch: as many per CU as HBM streams best with (wave_resident). So too the
+    // fused f32 radial steps of the two-buffer modes, 5 blocks of 256 threads per CU in identity-mapped launches
+    // of 2^24 elements or more. 1.2e8 elements, 8 / 7 / 6 / 5 / 4 / 3 per CU: T2 604.5 / 602.5 / 589.0 / 576.2
+    // / 583.7 / 647.8 us, CLM 566.0 / 560.3 / 554.7 / 548.1 / 573.2 / 599.1; T2 with 8 and 5 per CU at 4e7
+    // elements 198.4 and 193.9, at 1.6e7 87.1 and 85.6, at 8e6 57.3 and 58.9. TD-CLM and T1 gain under 1%
+    // (6 per CU) and keep 8.
+    const bool radial_limited = radial_f32 && identity_map && args.total_units >= kRadialLimitUnits &&
+                                (mode == LV_BUFFER_DUAL || mode == LV_BUFFER_T2);
+    uint32_t lds = 0;
+    if (threads < kThreads && (args.flags & kFLarge)) lds = wave_lds_bytes(wave_resident(mode, pt, (args.flags & kFMaster) != 0, table));
+    else if (radial_limited) lds = wave_lds_bytes(5);
     for (uint32_t ub = 0; ub < args.total_units; ub += std::min<uint32_t>(max_grid, args.total_units - ub)) {
         const uint32_t grid = std::min<uint32_t>(max_grid, args.total_units - ub);
         args.unit_base = ub;

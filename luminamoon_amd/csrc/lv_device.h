@@ -167,7 +167,7 @@ constexpr uint32_t wave_resident(int mode, int pt, bool master, bool table) {
     return mode == LV_BUFFER_T1 && !table ? 0u : 32u;
 }
 
-// Dynamic LDS bytes of a one-wave block that leave room for `resident` blocks on a CU: LDS is 160 KB
+// Dynamic LDS bytes of a block that leave room for `resident` blocks on a CU: LDS is 160 KB
 // in granules of 1280 bytes, and the kernel's own few bytes stay within the last granule.
 constexpr uint32_t wave_lds_bytes(uint32_t resident) { return resident && resident < 32u ? 128u / resident * 1280u - 256u : 0u; }
 

@@ -89,6 +89,31 @@ def test_two_pass_large_launches_match_oracle(buffer, pdt, sdt, extra, count):
     assert all(int(torch.count_nonzero(ws)) == 0 for ws in stepper.workspace._bufs.values())
 
 
+@pytest.mark.parametrize("sizes", [EDGES, EDGES * 3 + [70_003]], ids=["one-launch", "two-launches"])
+@pytest.mark.parametrize("buffer", [2, "T2"])
+def test_f32_radial_large_launches_match_oracle(buffer, sizes):
+    """Block b on unit b with fewer blocks per CU; the unit records and their fold keep unit order."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a ROCm GPU")
+    from luminamoon_amd.optimizer import hip_backend
+    from oracle import oracle as O
+
+    group = group_dict(buffer=buffer, lr=1e-3, bound_type="radial")
+    cfg = oracle_config(O, group)
+    host = TensorSet(sizes, "f32", "f32", "f32", True, False, 80)
+    dev, fill = _large(host)
+    stepper = hip_backend.HipStepper()
+    print(f"[case] radial {buffer} tensors={len(sizes)}", flush=True)
+    with O.radial_sum_f64():
+        for step in (1, 2, 3):
+            grads = host.grads(step, 80)
+            host.oracle_step(O, cfg, grads, step, threads=4)
+            dev.hip_step(stepper, group, [g.cuda() for g in grads] + [fill], step)
+            torch.cuda.synchronize()
+            host.assert_equal(dev, f"step {step}")
+    assert all(int(torch.count_nonzero(ws)) == 0 for ws in stepper.workspace._bufs.values())
+
+
 # Waves whose elements leave optimistic lanes' ranges: the kernels compute them again on the general path.
 def _exact_cancellation(host, grads):
     for m, g in zip(host.m, grads):  # m' or the direction near or at zero beside ordinary elements
