@@ -56,7 +56,7 @@ namespace lv {
 
 // ------------------------------------------------------------------ host side
 
-static KernelFn pick_kernel(int mode, int pt, int st, int pass, uint32_t flags, bool table) {
+static Kernel pick_kernel(int mode, int pt, int st, int pass, uint32_t flags, bool table) {
     switch (mode) {
     case LV_BUFFER_TDCLM: return pick_kernel_tdclm(pt, st, pass, flags, table);
     case LV_BUFFER_DUAL: return pick_kernel_clm(pt, st, pass, flags, table);
@@ -573,8 +573,8 @@ static int order_after(WsOrder *o, hipStream_t stream) {
 // (`radial_piece` for radial counting launches, the unit records of one piece; LV_MAX_GRID_BLOCKS
 // lowers the cap, so tests can split small launches). A counting launch folds its counts in its
 // last blocks; a radial one runs fold_kernel after every piece.
-static int launch(Args &args, int mode, int pt, int st, int pass, hipStream_t stream, bool table, uint32_t radial_piece) {
-    KernelFn fn = pick_kernel(mode, pt, st, pass, args.flags, table);
+static int launch(const Kernel &kernel, Args &args, int mode, int pt, int st, int pass, hipStream_t stream, bool table,
+                  uint32_t radial_piece) {
     const bool radial = (pass == kFused || pass == kCount) && (args.flags & kFRadial);
     if (table && radial) return fail(LV_STATUS_INVALID_CONFIG, "radial counting launches are inline");
     if (args.total_units == 0) return LV_STATUS_SUCCESS;
@@ -597,8 +597,7 @@ static int launch(Args &args, int mode, int pt, int st, int pass, hipStream_t st
                             args.flags == radial_flags(LV_DTYPE_F32) &&
                             (mode == LV_BUFFER_DUAL || mode == LV_BUFFER_T2 || args.total_units <= kRadialOneBufferUnits);
     const bool identity_map = st == LV_DTYPE_F32 && (!radial || radial_f32) &&
-                              (unit_threads(mode, pt, st, pass, args.flags, table) < kThreads ||
-                               args.total_units <= kIdentityMapUnits);
+                              (kernel.threads < kThreads || args.total_units <= kIdentityMapUnits);
     args.xcds = identity_map ? 1u : device_xcds();
     // b / X == (b * recip) >> 40 for b < 2^23 = kMaxGrid and X <= 64: recip exceeds 2^40 / X by at
     // most 1, so the product exceeds b * 2^40 / X by less than b < 2^23, i.e. by < 2^-17 after the
@@ -617,7 +616,6 @@ static int launch(Args &args, int mode, int pt, int st, int pass, hipStream_t st
     }
     if (max_grid == 0) return fail(LV_STATUS_INVALID_CONFIG, "no radial unit records in the workspace");
     KernelFn fold = radial ? pick_fold(mode, pass) : nullptr;
-    const uint32_t threads = unit_threads(mode, pt, st, pass, args.flags, table);
     // One-wave blocks of a large launch: as many per CU as HBM streams best with (wave_resident). So too the
     // fused f32 radial steps of the two-buffer modes, 5 blocks of 256 threads per CU in identity-mapped launches
     // of 2^24 elements or more. 1.2e8 elements, 8 / 7 / 6 / 5 / 4 / 3 per CU: T2 604.5 / 602.5 / 589.0 / 576.2
@@ -627,7 +625,8 @@ static int launch(Args &args, int mode, int pt, int st, int pass, hipStream_t st
     const bool radial_limited = radial_f32 && identity_map && args.total_units >= kRadialLimitUnits &&
                                 (mode == LV_BUFFER_DUAL || mode == LV_BUFFER_T2);
     uint32_t lds = 0;
-    if (threads < kThreads && (args.flags & kFLarge)) lds = wave_lds_bytes(wave_resident(mode, pt, (args.flags & kFMaster) != 0, table));
+    if (kernel.threads < kThreads && (kernel.flags & kFLarge))
+        lds = wave_lds_bytes(wave_resident(mode, pt, (kernel.flags & kFMaster) != 0, table));
     else if (radial_limited) lds = wave_lds_bytes(5);
     for (uint32_t ub = 0; ub < args.total_units; ub += std::min<uint32_t>(max_grid, args.total_units - ub)) {
         const uint32_t grid = std::min<uint32_t>(max_grid, args.total_units - ub);
@@ -635,7 +634,7 @@ static int launch(Args &args, int mode, int pt, int st, int pass, hipStream_t st
         args.piece_units = grid;
         args.xcd_q = grid / args.xcds;
         args.xcd_r = grid % args.xcds;
-        int rc = launch_one(fn, args, grid, threads, stream, lds);
+        int rc = launch_one(kernel.fn, args, grid, kernel.threads, stream, lds);
         if (rc != LV_STATUS_SUCCESS) return rc;
         if (radial) {
             uint32_t chunks = 0;
@@ -751,8 +750,9 @@ static bool lane_facts(const lv_config *cfg, const Args &args) {
     return args.b1sq >= 0x1p-20f && args.omb1sq >= 0x1p-20f && cfg->eps >= 0x1p-40f;
 }
 
-// `elems`: the elements of the launch's class.
-static void fill_args_common(Args &args, const lv_config *cfg, const Item &h, int bound, uint64_t elems, bool table) {
+// The launch arguments of a class's pass, but for its tensors, and the kernel that takes them (picked
+// once: the launch's units, blocks and threads are that kernel's). `elems`: the elements of the class.
+static Kernel fill_args_common(Args &args, const lv_config *cfg, const Item &h, int bound, uint64_t elems, bool table) {
     std::memset(&args, 0, sizeof args);
     args.lr = cfg->lr;
     args.b1 = cfg->beta1;
@@ -793,10 +793,10 @@ static void fill_args_common(Args &args, const lv_config *cfg, const Item &h, in
     // A counting pass without the radial bound reads neither the rounding, the decay, the bound nor the
     // master options: it takes the kernel of the reference defaults.
     if (h.pass == kCount && bound != LV_BOUND_RADIAL && cfg->cautious && h.gt == h.pt) flags = static_flags(h.pt, kCount);
-    if (elems >= kLargeElems && unit_large(cfg->buffer, h.pt, h.st, h.pass, flags, table) &&
-        (!unit_lanes(cfg->buffer, h.pt, h.st, h.pass, flags | kFLarge) || lane_facts(cfg, args)))
-        flags |= kFLarge;
     args.flags = flags;
+    const bool large = elems >= kLargeElems &&
+                       (!unit_lanes(cfg->buffer, h.pt, h.st, h.pass, flags | kFLarge) || lane_facts(cfg, args));
+    return pick_kernel(cfg->buffer, h.pt, h.st, h.pass, large ? flags | kFLarge : flags, table);
 }
 
 // An item's step count and first pass: dual.rs:52, dual.rs:122, dual.rs:260; tdclm.rs:67-68.
@@ -871,9 +871,9 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
             ph.pass = pi == 0 ? h.pass : (int)kApply;
             const int n = cls_end - begin;
             Args args;
-            fill_args_common(args, cfg, ph, bound, elems, table);
+            const Kernel kernel = fill_args_common(args, cfg, ph, bound, elems, table);
             args.step_rec = rec;
-            const uint32_t unit_elems = lv::unit_elems(cfg->buffer, ph.pt, ph.st, ph.pass, args.flags, true);
+            const uint32_t unit_elems = kernel.unit_elems;
             std::vector<TDesc> &tab = *tab_buf;
             if (tab.size() < (size_t)n) tab.resize((size_t)n);
             uint64_t units = 0, slot = 0;
@@ -904,7 +904,7 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
             int rc = acquire_table(tab.data(), (size_t)n, stream, lease);
             if (rc != LV_STATUS_SUCCESS) return rc;
             args.dtab = lease.s->dev;
-            rc = launch(args, cfg->buffer, ph.pt, ph.st, ph.pass, stream, true, 0);
+            rc = launch(kernel, args, cfg->buffer, ph.pt, ph.st, ph.pass, stream, true, 0);
             const int rr = release_table(lease, stream);
             if (rc != LV_STATUS_SUCCESS) return rc;
             if (rr != LV_STATUS_SUCCESS) return rr;
@@ -918,9 +918,9 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
             for (int pi = 0; pi < npass; pi++) {
                 ph.pass = pi == 0 ? h.pass : (int)kApply;
                 Args args;
-                fill_args_common(args, cfg, ph, bound, elems, table);
+                const Kernel kernel = fill_args_common(args, cfg, ph, bound, elems, table);
                 args.step_rec = rec;
-                const uint32_t unit_elems = lv::unit_elems(cfg->buffer, ph.pt, ph.st, ph.pass, args.flags, false);
+                const uint32_t unit_elems = kernel.unit_elems;
                 args.ndesc = end - begin;
                 uint64_t units = 0;
                 for (int k = begin; k < end; k++) {
@@ -942,7 +942,7 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
                 args.chunks = L.chunks;
                 args.unit_sq = L.unit_sq;
                 args.unit_cnt = L.unit_cnt;
-                const int rc = launch(args, cfg->buffer, ph.pt, ph.st, ph.pass, stream, false, L.radial_units);
+                const int rc = launch(kernel, args, cfg->buffer, ph.pt, ph.st, ph.pass, stream, false, L.radial_units);
                 if (rc != LV_STATUS_SUCCESS) return rc;
             }
             begin = end;

@@ -177,12 +177,14 @@ constexpr uint32_t wave_lds_bytes(uint32_t resident) { return resident && reside
 constexpr uint64_t kLargeElems = 1ull << 25;
 
 // Whether the kernels of this word have a form for large launches (kFLarge), with the reference
-// defaults: the passes that write the update, with f32 state and with or without a master copy, in
+// defaults: the passes that write the update, with f32 state and with or without a master copy (but
+// not the separate master of an f32 param, a rare call that keeps the ordinary kernels), in
 // one-wave blocks (wave_resident; non-cautious CLM f32 582.9 -> 536.4 us, 1.2e8 elements unfused);
 // the counting pass in larger units (unit_subs).
 constexpr bool unit_large(int mode, int pt, int st, int pass, uint32_t flags, bool table) {
     if (pass == kCount) return (flags & ~(uint32_t)kFLarge) == static_flags(pt, pass);
     if ((flags & ~(uint32_t)(kFMaster | kFLarge)) != static_flags(pt, pass)) return false;
+    if (pt == LV_DTYPE_F32 && (flags & kFMaster)) return false;
     const bool arithmetic = (mode == LV_BUFFER_DUAL || mode == LV_BUFFER_TDCLM) && pt != LV_DTYPE_F32 && !(flags & kFMaster);
     if (st != LV_DTYPE_F32 || arithmetic) return unit_lanes(mode, pt, st, pass, flags | kFLarge);
     return wave_resident(mode, pt, (flags & kFMaster) != 0, table) != 0;
@@ -2137,6 +2139,21 @@ __global__ void __launch_bounds__(kThreads) fold_kernel(const Args a) {
 
 using KernelFn = void (*)(Args);
 
+// A unit kernel with the launch geometry it was built for. Both come from one template word, so the
+// host cuts, sizes and launches what the kernel will read: nothing on the host works out a kernel's
+// threads or work unit from the option word of the call.
+struct Kernel {
+    KernelFn fn;
+    uint32_t flags;       // the kernel's template word (kFDynamic: options read from Args::flags)
+    uint32_t threads;     // per block
+    uint32_t unit_elems;  // elements per work unit
+};
+
+template <int MODE, int PT, int ST, int PASS, uint32_t FL, bool TABLE>
+Kernel kernel_of() {
+    return {unit_kernel<MODE, PT, ST, PASS, FL, TABLE>, FL, (uint32_t)unit_threads(MODE, PT, ST, PASS, FL, TABLE),
+            unit_elems(MODE, PT, ST, PASS, FL, TABLE)};
+}
 
 // The same defaults with bound_type="radial" (the radial passes never run SINGLE).
 constexpr uint32_t radial_flags(int PT) {
@@ -2144,33 +2161,35 @@ constexpr uint32_t radial_flags(int PT) {
             (PT == LV_DTYPE_F16 ? (uint32_t)kFClampV : 0u) | ((uint32_t)PT << 8));
 }
 
+// The kernel for an option word; kFLarge in it asks for the large form where there is one, else the
+// word's ordinary kernel is taken.
 // Table launches (many small tensors) have the reference defaults specialised too: on cfg2's 64
 // tensors the run-time-flag table kernel took 22.5 us per launch and the specialised one 19.2,
 // level with a memory-only twin (19.4).
 template <int MODE, int PT, int ST, int PASS>
-KernelFn pick_flags(uint32_t flags, bool table) {
+Kernel pick_flags(uint32_t flags, bool table) {
     constexpr uint32_t kStatic = static_flags(PT, PASS);
     constexpr uint32_t kRadial = radial_flags(PT);
-    if constexpr (PASS == kCount) {
-        constexpr uint32_t kL = kStatic | kFLarge;
-        if (flags == kL) return table ? unit_kernel<MODE, PT, ST, PASS, kL, true> : unit_kernel<MODE, PT, ST, PASS, kL, false>;
-    } else {  // the kernels of large launches
-        constexpr uint32_t kW = kStatic | kFLarge, kWM = kW | kFMaster;
-        if (flags == kW) {
-            if constexpr (unit_large(MODE, PT, ST, PASS, kW, true))
-                if (table) return unit_kernel<MODE, PT, ST, PASS, kW, true>;
-            if constexpr (unit_large(MODE, PT, ST, PASS, kW, false))
-                if (!table) return unit_kernel<MODE, PT, ST, PASS, kW, false>;
-        }
-        if constexpr (PT != LV_DTYPE_F32 && unit_large(MODE, PT, ST, PASS, kWM, true))
-            if (flags == kWM) return table ? unit_kernel<MODE, PT, ST, PASS, kWM, true> : unit_kernel<MODE, PT, ST, PASS, kWM, false>;
+    constexpr uint32_t kW = kStatic | kFLarge, kWM = kW | kFMaster;
+    if (flags == kW) {
+        if constexpr (unit_large(MODE, PT, ST, PASS, kW, true))
+            if (table) return kernel_of<MODE, PT, ST, PASS, kW, true>();
+        if constexpr (unit_large(MODE, PT, ST, PASS, kW, false))
+            if (!table) return kernel_of<MODE, PT, ST, PASS, kW, false>();
     }
+    if (flags == kWM) {
+        if constexpr (unit_large(MODE, PT, ST, PASS, kWM, true))
+            if (table) return kernel_of<MODE, PT, ST, PASS, kWM, true>();
+        if constexpr (unit_large(MODE, PT, ST, PASS, kWM, false))
+            if (!table) return kernel_of<MODE, PT, ST, PASS, kWM, false>();
+    }
+    flags &= ~(uint32_t)kFLarge;
     if (table) {
-        if (flags == kStatic) return unit_kernel<MODE, PT, ST, PASS, kStatic, true>;
-        return unit_kernel<MODE, PT, ST, PASS, kFDynamic, true>;
+        if (flags == kStatic) return kernel_of<MODE, PT, ST, PASS, kStatic, true>();
+        return kernel_of<MODE, PT, ST, PASS, kFDynamic, true>();
     }
-    if (flags == kStatic) return unit_kernel<MODE, PT, ST, PASS, kStatic, false>;
-    if (flags == kRadial) return unit_kernel<MODE, PT, ST, PASS, kRadial, false>;
+    if (flags == kStatic) return kernel_of<MODE, PT, ST, PASS, kStatic, false>();
+    if (flags == kRadial) return kernel_of<MODE, PT, ST, PASS, kRadial, false>();
     if constexpr (PASS == kFused) {
         // The steady step of common departures from the defaults: master weights, no stochastic
         // rounding, no weight decay. Where the step is VALU-bound the run-time-flag kernel costs
@@ -2178,15 +2197,15 @@ KernelFn pick_flags(uint32_t flags, bool table) {
         constexpr uint32_t kMaster = kStatic | kFMaster;
         constexpr uint32_t kNoSR = kStatic & ~(uint32_t)kFSR;
         constexpr uint32_t kNoWD = kStatic & ~(uint32_t)kFWeightDecay;
-        if (flags == kMaster) return unit_kernel<MODE, PT, ST, PASS, kMaster, false>;
-        if (flags == kNoSR) return unit_kernel<MODE, PT, ST, PASS, kNoSR, false>;
-        if (flags == kNoWD) return unit_kernel<MODE, PT, ST, PASS, kNoWD, false>;
+        if (flags == kMaster) return kernel_of<MODE, PT, ST, PASS, kMaster, false>();
+        if (flags == kNoSR) return kernel_of<MODE, PT, ST, PASS, kNoSR, false>();
+        if (flags == kNoWD) return kernel_of<MODE, PT, ST, PASS, kNoWD, false>();
     }
-    return unit_kernel<MODE, PT, ST, PASS, kFDynamic, false>;
+    return kernel_of<MODE, PT, ST, PASS, kFDynamic, false>();
 }
 
 template <int MODE, int PT, int ST>
-KernelFn pick_pass(int pass, uint32_t flags, bool table) {
+Kernel pick_pass(int pass, uint32_t flags, bool table) {
     switch (pass) {
     case kSingle: return pick_flags<MODE, PT, ST, kSingle>(flags, table);
     case kFused: return pick_flags<MODE, PT, ST, kFused>(flags, table);
@@ -2196,13 +2215,13 @@ KernelFn pick_pass(int pass, uint32_t flags, bool table) {
 }
 
 template <int MODE, int PT>
-KernelFn pick_state(int st, int pass, uint32_t flags, bool table) {
+Kernel pick_state(int st, int pass, uint32_t flags, bool table) {
     return st == LV_DTYPE_F32 ? pick_pass<MODE, PT, LV_DTYPE_F32>(pass, flags, table)
                               : pick_pass<MODE, PT, LV_DTYPE_BF16>(pass, flags, table);
 }
 
 template <int MODE>
-KernelFn pick_param(int pt, int st, int pass, uint32_t flags, bool table) {
+Kernel pick_param(int pt, int st, int pass, uint32_t flags, bool table) {
     switch (pt) {
     case LV_DTYPE_F32: return pick_state<MODE, LV_DTYPE_F32>(st, pass, flags, table);
     case LV_DTYPE_BF16: return pick_state<MODE, LV_DTYPE_BF16>(st, pass, flags, table);
@@ -2216,10 +2235,10 @@ KernelFn pick_fold_pass(int pass) {
 }
 
 // One per buffer mode, each defined in its own kernel unit (lv_kernels.hip built with LV_MODE).
-KernelFn pick_kernel_tdclm(int pt, int st, int pass, uint32_t flags, bool table);
-KernelFn pick_kernel_clm(int pt, int st, int pass, uint32_t flags, bool table);
-KernelFn pick_kernel_t1(int pt, int st, int pass, uint32_t flags, bool table);
-KernelFn pick_kernel_t2(int pt, int st, int pass, uint32_t flags, bool table);
+Kernel pick_kernel_tdclm(int pt, int st, int pass, uint32_t flags, bool table);
+Kernel pick_kernel_clm(int pt, int st, int pass, uint32_t flags, bool table);
+Kernel pick_kernel_t1(int pt, int st, int pass, uint32_t flags, bool table);
+Kernel pick_kernel_t2(int pt, int st, int pass, uint32_t flags, bool table);
 KernelFn pick_fold_tdclm(int pass);
 KernelFn pick_fold_clm(int pass);
 KernelFn pick_fold_t1(int pass);

@@ -10,22 +10,22 @@
 namespace lv {
 
 #if LV_MODE == LV_BUFFER_TDCLM
-KernelFn pick_kernel_tdclm(int pt, int st, int pass, uint32_t flags, bool table) {
+Kernel pick_kernel_tdclm(int pt, int st, int pass, uint32_t flags, bool table) {
     return pick_param<LV_BUFFER_TDCLM>(pt, st, pass, flags, table);
 }
 KernelFn pick_fold_tdclm(int pass) { return pick_fold_pass<LV_BUFFER_TDCLM>(pass); }
 #elif LV_MODE == LV_BUFFER_DUAL
-KernelFn pick_kernel_clm(int pt, int st, int pass, uint32_t flags, bool table) {
+Kernel pick_kernel_clm(int pt, int st, int pass, uint32_t flags, bool table) {
     return pick_param<LV_BUFFER_DUAL>(pt, st, pass, flags, table);
 }
 KernelFn pick_fold_clm(int pass) { return pick_fold_pass<LV_BUFFER_DUAL>(pass); }
 #elif LV_MODE == LV_BUFFER_T1
-KernelFn pick_kernel_t1(int pt, int st, int pass, uint32_t flags, bool table) {
+Kernel pick_kernel_t1(int pt, int st, int pass, uint32_t flags, bool table) {
     return pick_param<LV_BUFFER_T1>(pt, st, pass, flags, table);
 }
 KernelFn pick_fold_t1(int pass) { return pick_fold_pass<LV_BUFFER_T1>(pass); }
 #elif LV_MODE == LV_BUFFER_T2
-KernelFn pick_kernel_t2(int pt, int st, int pass, uint32_t flags, bool table) {
+Kernel pick_kernel_t2(int pt, int st, int pass, uint32_t flags, bool table) {
     return pick_param<LV_BUFFER_T2>(pt, st, pass, flags, table);
 }
 KernelFn pick_fold_t2(int pass) { return pick_fold_pass<LV_BUFFER_T2>(pass); }

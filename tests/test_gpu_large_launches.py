@@ -114,6 +114,34 @@ def test_f32_radial_large_launches_match_oracle(buffer, sizes):
     assert all(int(torch.count_nonzero(ws)) == 0 for ws in stepper.workspace._bufs.values())
 
 
+@pytest.mark.parametrize("count", [len(EDGES), 60], ids=["inline", "table"])
+@pytest.mark.parametrize("buffer,extra", [
+    (1, {}), (2, {}), ("T1", {}), ("T2", {}), (2, {"cautious": False}), ("T1", {"fused_single_pass": False}),
+])
+def test_f32_params_with_separate_masters_match_oracle(buffer, extra, count):
+    """An f32 param whose master copy is another buffer has no kernel of its own for large launches: the
+    ordinary one must be launched with its own units. Passes counting, applying, fused and single."""
+    if not torch.cuda.is_available():
+        pytest.skip("needs a ROCm GPU")
+    from luminamoon_amd.optimizer import hip_backend
+    from oracle import oracle as O
+
+    group = group_dict(buffer=buffer, lr=1e-3, master_weights="full", **extra)
+    cfg = oracle_config(O, group)
+    sizes = [EDGES[i % len(EDGES)] for i in range(count)]
+    host = TensorSet(sizes, "f32", "f32", "f32", buffer in (2, "T2"), True, 81)
+    dev, fill = _large(host)
+    stepper = hip_backend.HipStepper()
+    print(f"[case] f32 with master {buffer} {extra} tensors={count}", flush=True)
+    for step in (1, 2, 3):
+        grads = host.grads(step, 81)
+        host.oracle_step(O, cfg, grads, step, threads=4)
+        dev.hip_step(stepper, group, [g.cuda() for g in grads] + [fill], step)
+        torch.cuda.synchronize()
+        host.assert_equal(dev, f"step {step}")
+    assert all(int(torch.count_nonzero(ws)) == 0 for ws in stepper.workspace._bufs.values())
+
+
 # Waves whose elements leave optimistic lanes' ranges: the kernels compute them again on the general path.
 def _exact_cancellation(host, grads):
     for m, g in zip(host.m, grads):  # m' or the direction near or at zero beside ordinary elements
