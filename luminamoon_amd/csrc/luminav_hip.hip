@@ -626,7 +626,7 @@ static int launch(const Kernel &kernel, Args &args, int mode, int pt, int st, in
                                 (mode == LV_BUFFER_DUAL || mode == LV_BUFFER_T2);
     uint32_t lds = 0;
     if (kernel.threads < kThreads && (kernel.flags & kFLarge))
-        lds = wave_lds_bytes(wave_resident(mode, pt, (kernel.flags & kFMaster) != 0, table));
+        lds = wave_lds_bytes(wave_resident(mode, pt, (kernel.flags & kFMaster) != 0));
     else if (radial_limited) lds = wave_lds_bytes(5);
     for (uint32_t ub = 0; ub < args.total_units; ub += std::min<uint32_t>(max_grid, args.total_units - ub)) {
         const uint32_t grid = std::min<uint32_t>(max_grid, args.total_units - ub);
@@ -751,8 +751,10 @@ static bool lane_facts(const lv_config *cfg, const Args &args) {
 }
 
 // The launch arguments of a class's pass, but for its tensors, and the kernel that takes them (picked
-// once: the launch's units, blocks and threads are that kernel's). `elems`: the elements of the class.
-static Kernel fill_args_common(Args &args, const lv_config *cfg, const Item &h, int bound, uint64_t elems, bool table) {
+// once: the launch's units, blocks and threads are that kernel's). `elems`, `count`: the elements and
+// tensors of the class.
+static Kernel fill_args_common(Args &args, const lv_config *cfg, const Item &h, int bound, uint64_t elems, int count,
+                               bool table) {
     std::memset(&args, 0, sizeof args);
     args.lr = cfg->lr;
     args.b1 = cfg->beta1;
@@ -796,7 +798,10 @@ static Kernel fill_args_common(Args &args, const lv_config *cfg, const Item &h, 
     args.flags = flags;
     const bool large = elems >= kLargeElems &&
                        (!unit_lanes(cfg->buffer, h.pt, h.st, h.pass, flags | kFLarge) || lane_facts(cfg, args));
-    return pick_kernel(cfg->buffer, h.pt, h.st, h.pass, large ? flags | kFLarge : flags, table);
+    const Kernel k = pick_kernel(cfg->buffer, h.pt, h.st, h.pass, large ? flags | kFLarge : flags, table);
+    if (table && k.threads < kThreads && elems < (uint64_t)count * wave_table_mean(cfg->buffer, h.pt, h.master))
+        return pick_kernel(cfg->buffer, h.pt, h.st, h.pass, flags, table);
+    return k;
 }
 
 // An item's step count and first pass: dual.rs:52, dual.rs:122, dual.rs:260; tdclm.rs:67-68.
@@ -871,7 +876,7 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
             ph.pass = pi == 0 ? h.pass : (int)kApply;
             const int n = cls_end - begin;
             Args args;
-            const Kernel kernel = fill_args_common(args, cfg, ph, bound, elems, table);
+            const Kernel kernel = fill_args_common(args, cfg, ph, bound, elems, cls_end - begin, table);
             args.step_rec = rec;
             const uint32_t unit_elems = kernel.unit_elems;
             std::vector<TDesc> &tab = *tab_buf;
@@ -918,7 +923,7 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
             for (int pi = 0; pi < npass; pi++) {
                 ph.pass = pi == 0 ? h.pass : (int)kApply;
                 Args args;
-                const Kernel kernel = fill_args_common(args, cfg, ph, bound, elems, table);
+                const Kernel kernel = fill_args_common(args, cfg, ph, bound, elems, cls_end - begin, table);
                 args.step_rec = rec;
                 const uint32_t unit_elems = kernel.unit_elems;
                 args.ndesc = end - begin;

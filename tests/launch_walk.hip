@@ -234,9 +234,13 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
         check(s0 >= ws && s0 + nslots * lv::kSlotStride * 8 <= ws + ws_bytes, "count slots outside the workspace", &l);
         // the form for large launches exactly where the kernel has one
         const uint32_t base = k.fl & ~(uint32_t)lv::kFLarge;
-        const bool has_form = !(k.fl & lv::kFDynamic) && lv::unit_large(k.mode, k.pt, k.st, k.pass, base, k.table);
-        const bool large = k.fl != lv::kFDynamic && (k.fl & lv::kFLarge);
-        check(large == (has_form && all >= lv::kLargeElems), "the large form is taken on other launches", &l);
+        const bool master = c.master_weights && T[0].master_param;
+        const uint32_t wanted = base & lv::kFDynamic ? a.flags : base;  // a dynamic kernel may stand in for a large form
+        bool take = lv::unit_large(k.mode, k.pt, k.st, k.pass, wanted) && all >= lv::kLargeElems;
+        if (k.table && lv::unit_threads(k.mode, k.pt, k.st, k.pass, wanted | lv::kFLarge, true) == 64)
+            take = take && all >= T.size() * lv::wave_table_mean(k.mode, k.pt, master);
+        const bool large = (k.fl & lv::kFLarge) != 0;
+        check(large == take, "the large form is taken on other launches", &l);
         g_large += large;
         g_one_wave += l.threads == 64;
     }
@@ -271,8 +275,11 @@ int main(int argc, char **argv) {
         uint64_t last;
         const char *max_grid;
     } shapes[] = {
-        {"inline", 5, 0, nullptr},           {"table", 60, 0, nullptr},
-        {"inline large", 5, (1u << 25) + 7, nullptr}, {"table large", 60, (1u << 25) + 7, nullptr},
+        {"inline", 5, 0, nullptr},
+        {"table", 60, 0, nullptr},
+        {"inline large", 5, (1u << 25) + 7, nullptr},
+        {"table large", 60, (1u << 27) + 7, nullptr},
+        {"table of small tensors", 60, (1u << 25) + 7, nullptr},
         {"table split", 60, 0, "50"},
     };
     static const uint64_t sizes[] = {1, 300, 1025, 4097, 70001, 64 * 1024 + 1};

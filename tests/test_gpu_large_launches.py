@@ -1,5 +1,5 @@
 """The kernels of large launches (kFLarge): the one-wave kernels with f32 state, the counting pass in
-4096-element units with any state, optimistic lanes. A zero tensor of 2^25 elements on the device alone
+4096-element units with any state, optimistic lanes. A zero tensor of 2^27 elements on the device alone
 makes the launch large; the small tensors before it are compared. Sizes around the 256-element unit, the 1024 elements behind a count slot, the 64 slots and the
 4096-element unit, table and inline launches, with and without a master copy, against the oracle
 bit for bit (the arithmetic is the other kernels', so any difference is an addressing or count error)."""
@@ -14,7 +14,8 @@ from tests.test_gpu_special_values import GRAD_SPECIALS, M_SPECIALS, P_SPECIALS,
 pytestmark = pytest.mark.gpu
 
 EDGES = [1, 3, 255, 256, 257, 511, 1023, 1024, 1025, 4095, 4097, 8192 + 2049, 64 * 256, 64 * 1024 - 1, 64 * 1024 + 1, 70_001]
-LARGE = 1 << 25  # kLargeElems
+# At least kLargeElems, and with 60 tensors beside it a mean tensor that one-wave table launches ask for (wave_table_mean).
+LARGE = 1 << 27
 
 
 def _large(host):
