@@ -161,7 +161,8 @@ static int launch_one(KernelFn fn, const Args &args, uint32_t grid, uint32_t thr
     return LV_STATUS_SUCCESS;
 }
 
-static uint64_t units_of(uint64_t n, uint32_t unit_elems) { return (n + unit_elems - 1) / unit_elems; }
+// Work units of n elements; unit sizes are powers of two (a division costs a many-tensor call 5 ns a tensor).
+static uint64_t units_of(uint64_t n, uint32_t unit_elems) { return (n + unit_elems - 1) >> __builtin_ctz(unit_elems); }
 
 // Count slots a tensor of `units` work units takes in a table launch: its count slots and its fold
 // slot.
@@ -287,6 +288,7 @@ struct Layout {
     uint64_t table_slots = 0;    // table count slots available (0: no table launches)
     uint32_t radial_units = 0;   // unit records available: the largest radial launch piece
     bool radial_split = true;    // a radial launch above radial_units runs in pieces (else: refused)
+    bool may_be_large = true;    // false: the whole call has fewer than kLargeElems elements
 };
 
 constexpr size_t chunk_bytes(uint32_t radial_units) {
@@ -324,11 +326,12 @@ static Layout make_layout(char *ws, uint64_t table_slots, uint32_t radial_units)
 // What a call needs, from its tensors alone (an upper bound over every class the call forms):
 // table count slots when more than kMaxDesc tensors step, and radial unit records up to one piece
 // when the config uses the radial bound. Units are counted at 1024 elements, the smallest unit size of
-// radial launches and the one that table launches' count slots follow (launch_count_slots).
-static void call_needs(const lv_config *cfg, const lv_tensor *T, int count, uint64_t &table_slots, uint32_t &radial_units) {
+// radial launches and the one that table launches' count slots follow (launch_count_slots). Returns
+// those units.
+static uint64_t call_needs(const lv_config *cfg, const lv_tensor *T, int count, uint64_t &table_slots, uint32_t &radial_units) {
     table_slots = 0;
     radial_units = 0;
-    if (!cfg || !T || count <= 0) return;
+    if (!cfg || !T || count <= 0) return 0;
     const bool radial = cfg->bound && cfg->bound_ratio > 0.0f && cfg->bound_type == LV_BOUND_RADIAL;
     uint64_t units = 0, slots = 0;
     int active = 0;
@@ -341,6 +344,7 @@ static void call_needs(const lv_config *cfg, const lv_tensor *T, int count, uint
     }
     if (active > kMaxDesc && !radial) table_slots = slots;
     if (radial) radial_units = (uint32_t)std::min<uint64_t>(units, kRadialPiece);
+    return units;
 }
 
 // ------------------------------------------------------------------ descriptor tables
@@ -750,11 +754,9 @@ static bool lane_facts(const lv_config *cfg, const Args &args) {
     return args.b1sq >= 0x1p-20f && args.omb1sq >= 0x1p-20f && cfg->eps >= 0x1p-40f;
 }
 
-// The launch arguments of a class's pass, but for its tensors, and the kernel that takes them (picked
-// once: the launch's units, blocks and threads are that kernel's). `elems`, `count`: the elements and
-// tensors of the class.
-static Kernel fill_args_common(Args &args, const lv_config *cfg, const Item &h, int bound, uint64_t elems, int count,
-                               bool table) {
+// The launch arguments of a class, but for its tensors and each pass's option word. Returns the class's
+// option word.
+static uint32_t fill_args_common(Args &args, const lv_config *cfg, const Item &h, int bound) {
     std::memset(&args, 0, sizeof args);
     args.lr = cfg->lr;
     args.b1 = cfg->beta1;
@@ -792,16 +794,28 @@ static Kernel fill_args_common(Args &args, const lv_config *cfg, const Item &h, 
     if (bound == LV_BOUND_COORDINATE) flags |= kFCoordinate;
     if (bound == LV_BOUND_RADIAL) flags |= kFRadial;
     flags |= (uint32_t)h.gt << 8;
-    // A counting pass without the radial bound reads neither the rounding, the decay, the bound nor the
-    // master options: it takes the kernel of the reference defaults.
-    if (h.pass == kCount && bound != LV_BOUND_RADIAL && cfg->cautious && h.gt == h.pt) flags = static_flags(h.pt, kCount);
-    args.flags = flags;
+    return flags;
+}
+
+// One pass of a class: its kernel and its option word (Args::flags).
+struct PassPlan {
+    int pass;
+    uint32_t flags;
+    Kernel kernel;  // picked once: the launch's units, blocks and threads are this kernel's
+};
+
+// `word`: the class's option word; `elems`, `count`: its elements and tensors.
+static PassPlan plan_pass(const lv_config *cfg, const Args &args, const Item &h, int pass, uint32_t word, uint64_t elems,
+                          int count, bool table) {
+    PassPlan p;
+    p.pass = pass;
+    p.flags = word;
     const bool large = elems >= kLargeElems &&
-                       (!unit_lanes(cfg->buffer, h.pt, h.st, h.pass, flags | kFLarge) || lane_facts(cfg, args));
-    const Kernel k = pick_kernel(cfg->buffer, h.pt, h.st, h.pass, large ? flags | kFLarge : flags, table);
-    if (table && k.threads < kThreads && elems < (uint64_t)count * wave_table_mean(cfg->buffer, h.pt, h.master))
-        return pick_kernel(cfg->buffer, h.pt, h.st, h.pass, flags, table);
-    return k;
+                       (!unit_lanes(cfg->buffer, h.pt, h.st, pass, p.flags | kFLarge) || lane_facts(cfg, args));
+    p.kernel = pick_kernel(cfg->buffer, h.pt, h.st, pass, large ? p.flags | kFLarge : p.flags, table);
+    if (table && p.kernel.threads < kThreads && elems < (uint64_t)count * wave_table_mean(cfg->buffer, h.pt, h.master))
+        p.kernel = pick_kernel(cfg->buffer, h.pt, h.st, pass, p.flags, table);
+    return p;
 }
 
 // An item's step count and first pass: dual.rs:52, dual.rs:122, dual.rs:260; tdclm.rs:67-68.
@@ -867,87 +881,108 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
         const bool radial = bound == LV_BOUND_RADIAL && h.pass != kSingle;
         const bool table = !radial && L.table_slots > 0 && tab_buf && cls_end - begin > kMaxDesc;
         uint64_t elems = 0;
-        for (int k = begin; k < cls_end; k++) elems += tensors[items[k].idx].numel;
-        // A two-pass class runs its counting pass, then the applying pass, each with work units of its
-        // own kernel's size.
-        Item ph = h;  // the class, with the pass being launched
+        if (L.may_be_large)
+            for (int k = begin; k < cls_end; k++) elems += tensors[items[k].idx].numel;
+        Args args;
+        const uint32_t word = fill_args_common(args, cfg, h, bound);
+        args.step_rec = rec;
+        args.tickets = L.tickets;
+        // A two-pass class runs its counting pass, then the applying pass. Both take the same descriptors
+        // (and descriptor table) unless their kernels have work units of different sizes.
+        PassPlan plan[2];
         const int npass = h.pass == kCount ? 2 : 1;
-        for (int pi = 0; table && pi < npass; pi++) {
-            ph.pass = pi == 0 ? h.pass : (int)kApply;
-            const int n = cls_end - begin;
-            Args args;
-            const Kernel kernel = fill_args_common(args, cfg, ph, bound, elems, cls_end - begin, table);
-            args.step_rec = rec;
-            const uint32_t unit_elems = kernel.unit_elems;
+        const int count = cls_end - begin;
+        plan[0] = plan_pass(cfg, args, h, h.pass, word, elems, count, table);
+        if (npass == 2) {
+            plan[1] = plan_pass(cfg, args, h, kApply, word, elems, count, table);
+            // A counting pass without the radial bound reads neither the rounding, the decay, the bound nor
+            // the master options: it takes the kernel of the reference defaults, in a small class only if
+            // its units are the applying kernel's (T1 with 16-bit state and no weight decay, 100 tensors of
+            // 1e6 elements together: a second set of descriptors made the step 18.2 -> 20.0 us).
+            if (!radial && (word & kFCautious) && h.gt == h.pt) {
+                const PassPlan p = plan_pass(cfg, args, h, kCount, static_flags(h.pt, kCount), elems, count, table);
+                if ((p.kernel.flags & kFLarge) || p.kernel.unit_elems == plan[1].kernel.unit_elems) plan[0] = p;
+            }
+        }
+        if (table) {
+            const int n = count;
             std::vector<TDesc> &tab = *tab_buf;
             if (tab.size() < (size_t)n) tab.resize((size_t)n);
-            uint64_t units = 0, slot = 0;
-            for (int k = 0; k < n; k++) {
-                const lv_tensor &T = tensors[items[begin + k].idx];
-                TDesc &E = tab[(size_t)k];
-                std::memset(&E, 0, sizeof E);
-                fill_desc(E.d, T, items[begin + k], dual, unit_elems);
-                const uint64_t u = desc_units(E.d, unit_elems);
-                E.d.unit_begin = (uint32_t)units;
-                units += u;
-                if (units > 0xFFFFFFFFull) return fail(LV_STATUS_INVALID_CONFIG, "too many work units in one launch");
-                E.unit_end = (uint32_t)units;
-                E.slot_base = (uint32_t)slot;
-                slot += table_slots_of(u, unit_elems);
-            }
-            if (slot > L.table_slots)
-                return fail(LV_STATUS_INVALID_CONFIG, "workspace too small: %llu table count slots needed, %llu present",
-                            (unsigned long long)slot, (unsigned long long)L.table_slots);
+            args.slots = L.tslots;
             args.ndesc = n;
-            args.total_units = (uint32_t)units;
             args.group = (uint32_t)((n + kTableHeads - 1) / kTableHeads);
             args.nheads = (uint32_t)((n + args.group - 1) / args.group);
-            for (uint32_t hd = 0; hd < args.nheads; hd++) args.ubegin[hd] = tab[(size_t)hd * args.group].d.unit_begin;
-            args.slots = L.tslots;
-            args.tickets = L.tickets;
             TableLease lease;
-            int rc = acquire_table(tab.data(), (size_t)n, stream, lease);
-            if (rc != LV_STATUS_SUCCESS) return rc;
-            args.dtab = lease.s->dev;
-            rc = launch(kernel, args, cfg->buffer, ph.pt, ph.st, ph.pass, stream, true, 0);
+            int rc = LV_STATUS_SUCCESS;
+            for (int pi = 0; pi < npass && rc == LV_STATUS_SUCCESS; pi++) {
+                const uint32_t unit_elems = plan[pi].kernel.unit_elems;
+                if (pi == 0 || plan[pi - 1].kernel.unit_elems != unit_elems) {
+                    rc = release_table(lease, stream);
+                    if (rc != LV_STATUS_SUCCESS) return rc;
+                    uint64_t units = 0, slot = 0;
+                    for (int k = 0; k < n; k++) {
+                        const lv_tensor &T = tensors[items[begin + k].idx];
+                        TDesc &E = tab[(size_t)k];
+                        std::memset(&E, 0, sizeof E);
+                        fill_desc(E.d, T, items[begin + k], dual, unit_elems);
+                        const uint64_t u = desc_units(E.d, unit_elems);
+                        E.d.unit_begin = (uint32_t)units;
+                        units += u;
+                        if (units > 0xFFFFFFFFull)
+                            return fail(LV_STATUS_INVALID_CONFIG, "too many work units in one launch");
+                        E.unit_end = (uint32_t)units;
+                        E.slot_base = (uint32_t)slot;
+                        slot += table_slots_of(u, unit_elems);
+                    }
+                    if (slot > L.table_slots)
+                        return fail(LV_STATUS_INVALID_CONFIG,
+                                    "workspace too small: %llu table count slots needed, %llu present",
+                                    (unsigned long long)slot, (unsigned long long)L.table_slots);
+                    args.total_units = (uint32_t)units;
+                    for (uint32_t hd = 0; hd < args.nheads; hd++)
+                        args.ubegin[hd] = tab[(size_t)hd * args.group].d.unit_begin;
+                    rc = acquire_table(tab.data(), (size_t)n, stream, lease);
+                    if (rc != LV_STATUS_SUCCESS) return rc;
+                    args.dtab = lease.s->dev;
+                }
+                args.flags = plan[pi].flags;
+                rc = launch(plan[pi].kernel, args, cfg->buffer, h.pt, h.st, plan[pi].pass, stream, true, 0);
+            }
             const int rr = release_table(lease, stream);
             if (rc != LV_STATUS_SUCCESS) return rc;
             if (rr != LV_STATUS_SUCCESS) return rr;
-        }
-        if (table) {
             begin = cls_end;
             continue;
         }
+        args.slots = L.slots;
+        args.run = L.run;
+        args.chunks = L.chunks;
+        args.unit_sq = L.unit_sq;
+        args.unit_cnt = L.unit_cnt;
         while (begin < cls_end) {
             const int end = begin + std::min(cls_end - begin, kMaxDesc);
+            args.ndesc = end - begin;
             for (int pi = 0; pi < npass; pi++) {
-                ph.pass = pi == 0 ? h.pass : (int)kApply;
-                Args args;
-                const Kernel kernel = fill_args_common(args, cfg, ph, bound, elems, cls_end - begin, table);
-                args.step_rec = rec;
-                const uint32_t unit_elems = kernel.unit_elems;
-                args.ndesc = end - begin;
-                uint64_t units = 0;
-                for (int k = begin; k < end; k++) {
-                    Desc &D = args.d[k - begin];
-                    const lv_tensor &T = tensors[items[k].idx];
-                    fill_desc(D, T, items[k], dual, unit_elems);
-                    D.unit_begin = (uint32_t)units;
-                    units += desc_units(D, unit_elems);
-                    if (units > 0xFFFFFFFFull) return fail(LV_STATUS_INVALID_CONFIG, "too many work units in one launch");
+                const uint32_t unit_elems = plan[pi].kernel.unit_elems;
+                if (pi == 0 || plan[pi - 1].kernel.unit_elems != unit_elems) {
+                    uint64_t units = 0;
+                    for (int k = begin; k < end; k++) {
+                        Desc &D = args.d[k - begin];
+                        const lv_tensor &T = tensors[items[k].idx];
+                        fill_desc(D, T, items[k], dual, unit_elems);
+                        D.unit_begin = (uint32_t)units;
+                        units += desc_units(D, unit_elems);
+                        if (units > 0xFFFFFFFFull)
+                            return fail(LV_STATUS_INVALID_CONFIG, "too many work units in one launch");
+                    }
+                    args.total_units = (uint32_t)units;
+                    if (radial && units > L.radial_units && !L.radial_split)
+                        return fail(LV_STATUS_INVALID_CONFIG,
+                                    "radial launch of %llu work units exceeds the %u unit records of this entry point",
+                                    (unsigned long long)units, L.radial_units);
                 }
-                args.total_units = (uint32_t)units;
-                if (radial && units > L.radial_units && !L.radial_split)
-                    return fail(LV_STATUS_INVALID_CONFIG,
-                                "radial launch of %llu work units exceeds the %u unit records of this entry point",
-                                (unsigned long long)units, L.radial_units);
-                args.slots = L.slots;
-                args.tickets = L.tickets;
-                args.run = L.run;
-                args.chunks = L.chunks;
-                args.unit_sq = L.unit_sq;
-                args.unit_cnt = L.unit_cnt;
-                const int rc = launch(kernel, args, cfg->buffer, ph.pt, ph.st, ph.pass, stream, false, L.radial_units);
+                args.flags = plan[pi].flags;
+                const int rc = launch(plan[pi].kernel, args, cfg->buffer, h.pt, h.st, plan[pi].pass, stream, false, L.radial_units);
                 if (rc != LV_STATUS_SUCCESS) return rc;
             }
             begin = end;
@@ -1190,7 +1225,7 @@ int lv_step_multi(const lv_config *cfg, const lv_tensor *tensors, int count, voi
     if (((uintptr_t)workspace & 255u) != 0) return fail(LV_STATUS_INVALID_CONFIG, "workspace must be 256-byte aligned");
     uint64_t tslots;
     uint32_t runits;
-    call_needs(cfg, tensors, count, tslots, runits);
+    const uint64_t units = call_needs(cfg, tensors, count, tslots, runits);
     const size_t need = layout_bytes(tslots, runits);
     if (workspace_bytes < need)
         return fail(LV_STATUS_INVALID_CONFIG, "workspace too small: %zu < %zu (lv_workspace_bytes_for)", workspace_bytes,
@@ -1216,7 +1251,8 @@ int lv_step_multi(const lv_config *cfg, const lv_tensor *tensors, int count, voi
         cs.remember(cfg, tensors, count, nitems);
     }
     if (nitems == 0) return LV_STATUS_SUCCESS;
-    const Layout L = make_layout(static_cast<char *>(workspace), tslots, runits);
+    Layout L = make_layout(static_cast<char *>(workspace), tslots, runits);
+    L.may_be_large = units >= kLargeElems / kHalf;
     hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
     WsOrder *order = nullptr;
     rc = order_before(workspace, stream, order);

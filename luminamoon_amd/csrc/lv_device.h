@@ -115,7 +115,7 @@ constexpr int kLaneGroup = 2;  // elements of a lane whose arithmetic is interle
 // and 5249 -> 4972 us (CLM), of a 1.2e8-element f32 step 821 -> 774 us (CLM); 2048-element units 3089,
 // 5060 and 774. Small launches lose (3.5e6 elements 22.1 -> 23.5 us) and keep 1024 or 2048.
 constexpr int unit_subs(int mode, int pt, int st, int pass, uint32_t flags) {
-    if (pass == kCount) return (flags & kFLarge) ? 4 / unit_halves(mode, pt, st) : 1;
+    if (pass == kCount && (flags & kFLarge)) return 4 / unit_halves(mode, pt, st);
     return (mode == LV_BUFFER_T1 && st != LV_DTYPE_F32 && pt != LV_DTYPE_F32 && flags == static_flags(pt, pass)) ? 2 : 1;
 }
 
@@ -282,8 +282,8 @@ __host__ __device__ inline uint32_t table_count_slots(uint32_t units) {
 // launches keep the slot count of 1024-element units (the workspace is sized for those): their slots
 // see up to 256 blocks.
 __host__ __device__ inline uint32_t launch_count_slots(uint32_t units, uint32_t unit_elems, bool table) {
-    const uint32_t r = table && unit_elems < kHalf ? kHalf / unit_elems : 1u;
-    return table_count_slots((units + r - 1u) / r);
+    const int sh = table && unit_elems < kHalf ? __builtin_ctz(kHalf) - __builtin_ctz(unit_elems) : 0;
+    return table_count_slots((units + (1u << sh) - 1u) >> sh);
 }
 
 // Radial-bound sums of a run of units: sum u_eff^2, sum p^2 (f64), mask count.

@@ -172,7 +172,7 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
     const bool two = c.fused_single_pass == 0 || (entry != kGraph && step < 2);
     const int first = (!c.cautious && bound != LV_BOUND_RADIAL) ? lv::kSingle : two ? lv::kCount : lv::kFused;
     std::map<const void *, int> seen[4];  // per pass: how often each param was stepped
-    uint32_t next = 0;
+    uint32_t next = 0, counted = 0;
     for (const Launch &l : g_launches) {
         if (!l.k.unit) continue;
         g_checked++;
@@ -229,6 +229,9 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
         }
         if (!ok) continue;
         check(units == a.total_units, "total units", &l);
+        // a small two-pass class cuts its tensors (and uploads its table) once for both passes
+        if (k.pass == lv::kCount) counted = unit;
+        if (k.pass == lv::kApply && all < lv::kLargeElems) check(unit == counted, "the passes' units differ", &l);
         const char *s0 = (const char *)a.slots;
         const uint64_t nslots = k.table ? slots : (uint64_t)a.ndesc * lv::kSlotWords;
         check(s0 >= ws && s0 + nslots * lv::kSlotStride * 8 <= ws + ws_bytes, "count slots outside the workspace", &l);
