@@ -804,7 +804,7 @@ struct PassPlan {
     Kernel kernel;  // picked once: the launch's units, blocks and threads are this kernel's
 };
 
-// `word`: the class's option word; `elems`, `count`: its elements and tensors.
+// `word`: the class's option word; `elems`, `count`: the elements and tensors of the launch.
 static PassPlan plan_pass(const lv_config *cfg, const Args &args, const Item &h, int pass, uint32_t word, uint64_t elems,
                           int count, bool table) {
     PassPlan p;
@@ -880,9 +880,6 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
         while (cls_end < nitems && same_class(items[cls_end], h)) cls_end++;
         const bool radial = bound == LV_BOUND_RADIAL && h.pass != kSingle;
         const bool table = !radial && L.table_slots > 0 && tab_buf && cls_end - begin > kMaxDesc;
-        uint64_t elems = 0;
-        if (L.may_be_large)
-            for (int k = begin; k < cls_end; k++) elems += tensors[items[k].idx].numel;
         Args args;
         const uint32_t word = fill_args_common(args, cfg, h, bound);
         args.step_rec = rec;
@@ -891,21 +888,26 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
         // (and descriptor table) unless their kernels have work units of different sizes.
         PassPlan plan[2];
         const int npass = h.pass == kCount ? 2 : 1;
-        const int count = cls_end - begin;
-        plan[0] = plan_pass(cfg, args, h, h.pass, word, elems, count, table);
-        if (npass == 2) {
-            plan[1] = plan_pass(cfg, args, h, kApply, word, elems, count, table);
+        // The kernels of one launch (or pair): the class's in a table launch, else those of a group of at
+        // most kMaxDesc of its tensors, whose own elements decide whether it is large.
+        const auto plan_launch = [&](int lo, int hi) {
+            uint64_t elems = 0;
+            if (L.may_be_large)
+                for (int k = lo; k < hi; k++) elems += tensors[items[k].idx].numel;
+            plan[0] = plan_pass(cfg, args, h, h.pass, word, elems, hi - lo, table);
+            if (npass == 1) return;
+            plan[1] = plan_pass(cfg, args, h, kApply, word, elems, hi - lo, table);
             // A counting pass without the radial bound reads neither the rounding, the decay, the bound nor
-            // the master options: it takes the kernel of the reference defaults, in a small class only if
+            // the master options: it takes the kernel of the reference defaults, in a small launch only if
             // its units are the applying kernel's (T1 with 16-bit state and no weight decay, 100 tensors of
             // 1e6 elements together: a second set of descriptors made the step 18.2 -> 20.0 us).
-            if (!radial && (word & kFCautious) && h.gt == h.pt) {
-                const PassPlan p = plan_pass(cfg, args, h, kCount, static_flags(h.pt, kCount), elems, count, table);
-                if ((p.kernel.flags & kFLarge) || p.kernel.unit_elems == plan[1].kernel.unit_elems) plan[0] = p;
-            }
-        }
+            if (radial || !(word & kFCautious) || h.gt != h.pt) return;
+            const PassPlan p = plan_pass(cfg, args, h, kCount, static_flags(h.pt, kCount), elems, hi - lo, table);
+            if ((p.kernel.flags & kFLarge) || p.kernel.unit_elems == plan[1].kernel.unit_elems) plan[0] = p;
+        };
         if (table) {
-            const int n = count;
+            const int n = cls_end - begin;
+            plan_launch(begin, cls_end);
             std::vector<TDesc> &tab = *tab_buf;
             if (tab.size() < (size_t)n) tab.resize((size_t)n);
             args.slots = L.tslots;
@@ -962,6 +964,7 @@ static int run_call(const lv_config *cfg, const lv_tensor *tensors, Item *items,
         while (begin < cls_end) {
             const int end = begin + std::min(cls_end - begin, kMaxDesc);
             args.ndesc = end - begin;
+            plan_launch(begin, end);
             for (int pi = 0; pi < npass; pi++) {
                 const uint32_t unit_elems = plan[pi].kernel.unit_elems;
                 if (pi == 0 || plan[pi - 1].kernel.unit_elems != unit_elems) {

@@ -194,7 +194,7 @@ constexpr uint64_t wave_table_mean(int mode, int pt, bool master) {
 // in granules of 1280 bytes, and the kernel's own few bytes stay within the last granule.
 constexpr uint32_t wave_lds_bytes(uint32_t resident) { return resident && resident < 32u ? 128u / resident * 1280u - 256u : 0u; }
 
-// Smallest launch (elements of its class) that takes the kernels' large forms (unit_large). Below it
+// Smallest launch, in elements, that takes the kernels' large forms (unit_large). Below it
 // a CU sees each of its waves only a few times and the limit costs what the order gains: at 4e6
 // elements 0.91-1.02x, at 8e6 0.97-1.02x, at 1.6e7 0.99-1.03x, at 3.2e7 1.01-1.05x (CLM f32, T2 bf16).
 constexpr uint64_t kLargeElems = 1ull << 25;

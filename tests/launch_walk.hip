@@ -189,7 +189,7 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
         next = a.unit_base + l.grid;
         check(next <= a.total_units, "blocks past the last unit", &l);
         if (next == a.total_units) next = 0;
-        uint64_t units = 0, slots = 0;
+        uint64_t units = 0, slots = 0, elems = 0;
         bool ok = true;
         for (int i = 0; i < a.ndesc && ok; i++) {
             const lv::Desc &D = k.table ? a.dtab[i].d : a.d[i];
@@ -213,6 +213,7 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
             const uint64_t u = (t.numel - (D.vec ? D.head : 0) + unit - 1) / unit;
             ok = ok && check(D.unit_begin == units, "units are not the kernel's", &l);
             units += u;
+            elems += t.numel;
             if (k.table) {  // the count slots and the fold slot the kernel will use
                 ok = ok && check(a.dtab[i].unit_end == units, "unit end", &l);
                 ok = ok && check(a.dtab[i].slot_base >= slots, "count slots of two tensors overlap", &l);
@@ -229,9 +230,9 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
         }
         if (!ok) continue;
         check(units == a.total_units, "total units", &l);
-        // a small two-pass class cuts its tensors (and uploads its table) once for both passes
+        // a small two-pass launch cuts its tensors (and uploads its table) once for both passes
         if (k.pass == lv::kCount) counted = unit;
-        if (k.pass == lv::kApply && all < lv::kLargeElems) check(unit == counted, "the passes' units differ", &l);
+        if (k.pass == lv::kApply && elems < lv::kLargeElems) check(unit == counted, "the passes' units differ", &l);
         const char *s0 = (const char *)a.slots;
         const uint64_t nslots = k.table ? slots : (uint64_t)a.ndesc * lv::kSlotWords;
         check(s0 >= ws && s0 + nslots * lv::kSlotStride * 8 <= ws + ws_bytes, "count slots outside the workspace", &l);
@@ -239,9 +240,9 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
         const uint32_t base = k.fl & ~(uint32_t)lv::kFLarge;
         const bool master = c.master_weights && T[0].master_param;
         const uint32_t wanted = base & lv::kFDynamic ? a.flags : base;  // a dynamic kernel may stand in for a large form
-        bool take = lv::unit_large(k.mode, k.pt, k.st, k.pass, wanted) && all >= lv::kLargeElems;
+        bool take = lv::unit_large(k.mode, k.pt, k.st, k.pass, wanted) && elems >= lv::kLargeElems;
         if (k.table && lv::unit_threads(k.mode, k.pt, k.st, k.pass, wanted | lv::kFLarge, true) == 64)
-            take = take && all >= T.size() * lv::wave_table_mean(k.mode, k.pt, master);
+            take = take && elems >= (uint64_t)a.ndesc * lv::wave_table_mean(k.mode, k.pt, master);
         const bool large = (k.fl & lv::kFLarge) != 0;
         check(large == take, "the large form is taken on other launches", &l);
         g_large += large;
