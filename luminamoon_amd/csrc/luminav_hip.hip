@@ -748,7 +748,13 @@ static uint64_t desc_units(const Desc &D, uint32_t unit_elems) {
 // The facts about the hyper-parameters that optimistic lanes (lane_update) rely on. They hold for
 // every step: beta1's bias correction lies in [1 - beta1^2, 1] and beta2's in (0, 1], so c1 and c2 are
 // at least their first factors below. `args` has the derived constants.
+// The first line keeps launches off the lanes whose waves would mostly fail their range test and be
+// computed twice (0.42-0.61x). The cautious scale lies in [1, 1 / clamp_min], so from lr 2^-30 on a step
+// falls under kLaneMinStep only for |u| < 3.1e-5 (1e8 elements against the general path: lr 0 0.42-0.61x,
+// 1e-12 0.43-1.05x, 1e-10 0.72-1.09x, 1e-9 1.01-1.09x, 1e-8 and up 1.03-1.14x), and up to 2^40 * clamp_min
+// lane_min_u has a bound.
 static bool lane_facts(const lv_config *cfg, const Args &args) {
+    if (!(cfg->lr >= 0x1p-30f) || !(cfg->lr <= 0x1p40f * cfg->cautious_clamp_min)) return false;
     if (!(args.ranges & kRangeM) || !(args.ranges & kRangeP) || !(cfg->bound_ratio >= 0x1p-20f)) return false;
     if (cfg->buffer == LV_BUFFER_DUAL) return args.omb1sq * cfg->tau * cfg->eps >= 1.1e-12f;
     return args.b1sq >= 0x1p-20f && args.omb1sq >= 0x1p-20f && cfg->eps >= 0x1p-40f;

@@ -239,10 +239,13 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
         // the form for large launches exactly where the kernel has one
         const uint32_t base = k.fl & ~(uint32_t)lv::kFLarge;
         const bool master = c.master_weights && T[0].master_param;
+        const bool lanes = lv::unit_lanes(k.mode, k.pt, k.st, k.pass, base | lv::kFLarge);
         const uint32_t wanted = base & lv::kFDynamic ? a.flags : base;  // a dynamic kernel may stand in for a large form
         bool take = lv::unit_large(k.mode, k.pt, k.st, k.pass, wanted) && elems >= lv::kLargeElems;
         if (k.table && lv::unit_threads(k.mode, k.pt, k.st, k.pass, wanted | lv::kFLarge, true) == 64)
             take = take && elems >= (uint64_t)a.ndesc * lv::wave_table_mean(k.mode, k.pt, master);
+        // lanes take no launch whose steps would mostly fall below their range
+        if (lanes) take = take && c.lr >= 0x1p-30f;
         const bool large = (k.fl & lv::kFLarge) != 0;
         check(large == take, "the large form is taken on other launches", &l);
         g_large += large;
@@ -303,13 +306,14 @@ int main(int argc, char **argv) {
                 const uint64_t n = sh.last && i == sh.count - 1 ? sh.last : sizes[(size_t)i % 6];
                 T.push_back(tensor(i, n, pt, gt, st, dual, master, offs[i % 5], goffs[i % 5]));
             }
-            for (int opt = 0; opt < 8; opt++)
+            for (float lr : {1e-3f, 9.5e-10f, 9e-10f, 0.0f})
+            for (int opt = lr == 1e-3f ? 0 : 7; opt < 8; opt++)
             for (int bound = 0; bound < 3; bound++)
             for (int when = 0; when < 3; when++)
             for (int entry = 0; entry < 3; entry++) {
                 lv_config c;
                 std::memset(&c, 0, sizeof c);
-                c.lr = 1e-3f; c.beta1 = 0.9f; c.beta2 = 0.999f; c.eps = 1e-8f; c.tau = 0.8f; c.lam = 0.3f;
+                c.lr = lr; c.beta1 = 0.9f; c.beta2 = 0.999f; c.eps = 1e-8f; c.tau = 0.8f; c.lam = 0.3f;
                 c.cautious_clamp_min = 0.5f; c.bound_ratio = 0.05f; c.ema_decay = 0.8f;
                 c.buffer = mode;
                 c.cautious = opt & 1;
@@ -322,7 +326,7 @@ int main(int argc, char **argv) {
                 c.seed = 1337;
                 g_case = std::string(sh.name) + " mode " + std::to_string(mode) + " params " + std::to_string(pt) + " grads " +
                          std::to_string(gt) + " state " + std::to_string(st) + " master " + std::to_string(master) +
-                         " options " + std::to_string(opt) + " bound " + std::to_string(bound) + " when " +
+                         " lr " + std::to_string(lr) + " options " + std::to_string(opt) + " bound " + std::to_string(bound) + " when " +
                          std::to_string(when) + " entry " + std::to_string(entry);
                 check_call(c, T, (Entry)entry, when == 0 ? 1 : 2, kRadialLimit);
             }
