@@ -692,8 +692,9 @@ static bool head_for(const lv_tensor &T, const Item &it, bool dual, uint32_t ali
 // at which every stream starts a whole unit of its own element size, that is at an element index
 // (address / element size) that is a multiple of kMinUnitElems, so each block moves the same
 // whole 512-byte (16-bit) and 1 KiB (f32) pieces of its streams as in an aligned tensor. A view
-// at +k elements of aligned buffers has h = 256 - k. Against the 128-byte-line head, a 2^27-element
-// T2 view at +1, +33 and +63 elements ran 1.033-1.037x the aligned view in one-wave blocks.
+// at +k elements of aligned buffers has h = 256 - k. 2^27-element views at +1, +17, +33, +130 and +200
+// against the aligned tensor, in one process: with these heads T2 bf16 1.004-1.017x, CLM, T2 and TD-CLM in
+// f32 0.98-1.02x; from the first 128-byte line 1.01-1.04x and 1.00-1.04x.
 static bool unit_head(const lv_tensor &T, const Item &it, bool dual, uint32_t &head) {
     struct Stream {
         uintptr_t addr;

@@ -243,24 +243,24 @@ struct Desc {
     void *v;
     float *mp;
     float *scratch;
-    uint64_t n;
+    uint64_t n : 63;    // elements (at most 2^40)
+    // vec: every stream is aligned at element `head` (one-wave kernels: at most 255 elements, to whole
+    // 256-element pieces of every stream where the views allow it; others: at most 63, to a 128-byte line;
+    // else to 16 bytes), so the tensor's work units start there and whole units take the vector path; the
+    // `head` elements before it are taken by one block (unit_kernel's takes_head). Set by the host from
+    // the pointers.
+    uint64_t vec : 1;
     uint32_t unit_begin;  // first work unit of this tensor in the launch's unit space
     uint32_t pidx;        // low 32 bits of param_index (seeds only need idx * 10007 mod 2^31)
     uint32_t ibase;       // low 32 bits of index_base (the SR offset is taken mod 2^32)
     uint32_t nskip : 24;  // inactive [begin, end) ranges in `skip` (sorted, disjoint)
-    // vec: every stream is aligned at element `head` (< 64; to a 128-byte line where the views
-    // allow it, else to 16 bytes), so the tensor's work units start there and whole units take
-    // the vector path; the `head` elements before it are taken one per thread by the block of the
-    // tensor's last unit. Set by the host from the pointers.
-    uint32_t head : 6;
-    uint32_t vec : 1;
-    uint32_t : 1;
+    uint32_t head : 8;
     const uint64_t *skip;
 };
 
 // A tensor of a table launch, in device memory: its descriptor, the end of its unit range and the
 // first of its count slots (64-byte slot index into Args::slots; the tensor has
-// table_count_slots(units) slots and one fold slot after them).
+// launch_count_slots(units) slots and one fold slot after them).
 struct TDesc {
     Desc d;
     uint32_t unit_end;
@@ -329,6 +329,7 @@ struct Args {
 constexpr int kTableHeads = kMaxDesc * (int)(sizeof(Desc) / sizeof(uint32_t));  // 960
 
 static_assert(sizeof(Desc) == 80, "descriptor layout");
+static_assert(kMinUnitElems - 1 < (1u << 8), "heads of one-wave kernels fit Desc::head");
 static_assert(sizeof(TDesc) == 88, "table descriptor layout");
 static_assert(sizeof(Args) <= 4096, "kernel arguments must fit in 4 KiB");
 
@@ -1943,10 +1944,9 @@ __global__ void __launch_bounds__(unit_threads(MODE, PT, ST, PASS, FL, TABLE), u
     // units start at the tensor's first 16-byte aligned element (tv.head > 0: an unaligned view)
     const uint64_t ubase = (uint64_t)(unit - tv.t_begin) * kUnit + tv.head;
     // Whether this block also takes the head. One-wave kernels (identity-mapped, heads of up to 255
-    // elements) use the tensor's first unit, whose block starts early in the launch: with the last
-    // unit, whose head round trips fall on the launch's tail, a 2^27-element T2 view at +1
-    // element ran 1.030x the aligned view, with the first 1.022x (and with the head spread over
-    // the first units' blocks, 64 elements each, 1.036x). The others keep the last unit, which
+    // elements) use the tensor's first unit, whose block starts early in the launch: the last unit's
+    // head round trips would fall on the launch's tail (heads of 63 elements of a 2^27-element T2
+    // view: last unit 1.030x the aligned view, first 1.022x). The others keep the last unit, which
     // also keeps the radial sums' fold order. Only after open_step: tv.t_end is set there.
     const auto takes_head = [&]() {
         if constexpr (TPB == kThreads) return tv.head && unit + 1u == tv.t_end;

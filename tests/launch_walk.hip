@@ -209,6 +209,13 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
                 if (D.v) al = al && ((uintptr_t)D.v + h * bytes_of(t.state_dtype)) % 16 == 0;
                 if (D.mp) al = al && ((uintptr_t)D.mp + h * 4) % 16 == 0;
                 ok = ok && check(al && h < t.numel, "vector layout from an unaligned element", &l);
+                // one-wave kernels: whole units of every stream, where the streams agree on an offset and the
+                // tensor reaches that far
+                const uintptr_t e = (uintptr_t)D.p / bytes_of(t.param_dtype) % 256;
+                bool same = (uintptr_t)D.g / bytes_of(t.grad_dtype) % 256 == e && (uintptr_t)D.m / bytes_of(t.state_dtype) % 256 == e;
+                same = same && (!D.v || (uintptr_t)D.v / bytes_of(t.state_dtype) % 256 == e) && (!D.mp || (uintptr_t)D.mp / 4 % 256 == e);
+                if (unit == 256 && same && (256 - e) % 256 < t.numel)
+                    ok = ok && check(h == (256 - e) % 256, "a one-wave kernel's units do not start at whole units", &l);
             }
             const uint64_t u = (t.numel - (D.vec ? D.head : 0) + unit - 1) / unit;
             ok = ok && check(D.unit_begin == units, "units are not the kernel's", &l);
