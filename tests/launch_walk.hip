@@ -266,6 +266,36 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
     }
 }
 
+static lv_config defaults(int mode, float lr, bool master) {
+    lv_config c;
+    std::memset(&c, 0, sizeof c);
+    c.lr = lr; c.beta1 = 0.9f; c.beta2 = 0.999f; c.eps = 1e-8f; c.tau = 0.8f; c.lam = 0.3f;
+    c.cautious_clamp_min = 0.5f; c.bound_ratio = 0.05f; c.ema_decay = 0.8f;
+    c.buffer = mode;
+    c.master_weights = master ? 2 : 0;
+    c.seed = 1337;
+    return c;
+}
+
+// route MODE PARAMS STATE MASTER SIZE...: the kernels of one fused step with the default options over
+// tensors of these sizes, one "flags threads" line per launch.
+static int route(int argc, char **argv) {
+    const int mode = std::atoi(argv[3]), pt = std::atoi(argv[4]), st = std::atoi(argv[5]);
+    const bool master = std::atoi(argv[6]) != 0;
+    lv_config c = defaults(mode, 1e-3f, master);
+    c.cautious = c.stochastic_rounding = c.bound = c.fused_single_pass = 1;
+    c.weight_decay = 0.1f;
+    c.bound_type = LV_BOUND_COORDINATE;
+    std::vector<lv_tensor> T;
+    for (int i = 7; i < argc; i++)
+        T.push_back(tensor(i - 7, std::strtoull(argv[i], nullptr, 10), pt, pt, st, mode == LV_BUFFER_DUAL || mode == LV_BUFFER_T2,
+                           master, 0, 0));
+    check_call(c, T, kMulti, 2, ~0ull);
+    for (const Launch &l : g_launches)
+        if (l.k.unit) std::printf("%u %u\n", l.k.fl, l.threads);
+    return g_bad ? 1 : 0;
+}
+
 int main(int argc, char **argv) {
     if (argc < 2) return 2;
     void *h = dlopen(argv[1], RTLD_NOW | RTLD_LOCAL);
@@ -282,6 +312,7 @@ int main(int argc, char **argv) {
         std::printf("the library's kernels were not registered with this program\n");
         return 2;
     }
+    if (argc > 6 && !std::strcmp(argv[2], "route")) return route(argc, argv);
     const uint64_t kRadialLimit = 1u << 16;
     struct Shape {
         const char *name;
@@ -318,19 +349,13 @@ int main(int argc, char **argv) {
             for (int bound = 0; bound < 3; bound++)
             for (int when = 0; when < 3; when++)
             for (int entry = 0; entry < 3; entry++) {
-                lv_config c;
-                std::memset(&c, 0, sizeof c);
-                c.lr = lr; c.beta1 = 0.9f; c.beta2 = 0.999f; c.eps = 1e-8f; c.tau = 0.8f; c.lam = 0.3f;
-                c.cautious_clamp_min = 0.5f; c.bound_ratio = 0.05f; c.ema_decay = 0.8f;
-                c.buffer = mode;
+                lv_config c = defaults(mode, lr, master);
                 c.cautious = opt & 1;
                 c.stochastic_rounding = (opt >> 1) & 1;
                 c.weight_decay = (opt & 4) ? 0.1f : 0.0f;
                 c.bound = bound != LV_BOUND_NONE;
                 c.bound_type = bound;
-                c.master_weights = master ? 2 : 0;
                 c.fused_single_pass = when != 2;
-                c.seed = 1337;
                 g_case = std::string(sh.name) + " mode " + std::to_string(mode) + " params " + std::to_string(pt) + " grads " +
                          std::to_string(gt) + " state " + std::to_string(st) + " master " + std::to_string(master) +
                          " lr " + std::to_string(lr) + " options " + std::to_string(opt) + " bound " + std::to_string(bound) + " when " +

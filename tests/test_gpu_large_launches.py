@@ -1,8 +1,10 @@
 """The kernels of large launches (kFLarge): the one-wave kernels with f32 state, the counting pass in
 4096-element units with any state, optimistic lanes. A zero tensor of 2^27 elements on the device alone
-makes the launch large; the small tensors before it are compared. Sizes around the 256-element unit, the 1024 elements behind a count slot, the 64 slots and the
-4096-element unit, table and inline launches, with and without a master copy, against the oracle
-bit for bit (the arithmetic is the other kernels', so any difference is an addressing or count error)."""
+makes the launch large (tests/test_launch_geometry.py checks on the CPU that it does); the small tensors
+beside it are compared. Sizes around the 256-element unit, the 1024 elements behind a count slot, the 64
+slots and the 4096-element unit, in table and inline launches, with and without a master copy; views,
+inactive ranges, shard offsets, single passes, split launches and graph steps. Against the oracle bit for
+bit (the arithmetic is the other kernels', so any difference is an addressing or count error)."""
 from __future__ import annotations
 
 import pytest
@@ -208,3 +210,166 @@ def test_optimistic_lanes_match_oracle(buffer, pdt, sdt, inputs):
                     a, b = getattr(host, name)[i], getattr(dev, name)[i]
                     if a is not None:
                         _assert_same(a, b, f"{extra} step {step} {name}[{i}]")
+
+
+# One of every large form: f32 state with and without a master, lanes with f32 and with 16-bit state.
+FORMS = [
+    (1, "f32", "f32", {}), (2, "f32", "f32", {}), ("T1", "f32", "f32", {}), ("T2", "f32", "f32", {}),
+    ("T2", "bf16", "f32", {}), ("T2", "f16", "f32", {}),
+    (2, "bf16", "f32", {"master_weights": "full"}), ("T2", "f16", "f32", {"master_weights": "semi"}),
+    ("T1", "bf16", "f32", {"master_weights": "full"}), (1, "f16", "f32", {"master_weights": "full"}),
+    (2, "bf16", "f32", {}), (2, "f16", "f32", {}), (1, "bf16", "f32", {}), (1, "f16", "f32", {}),
+    (2, "bf16", "bf16", {"state_precision": "param"}), (1, "bf16", "bf16", {"state_precision": "param"}),
+]
+FORM_IDS = ["-".join(map(str, f[:3])) + ("-master" if "master_weights" in f[3] else "") for f in FORMS]
+
+
+class _Case:
+    """A form's tensors on the host and on the device, the device's as views at `offs` elements into their
+    buffers and with one zero tensor of LARGE elements behind them; steps both and compares."""
+
+    def __init__(self, form, sizes, offs=None, ranges=None, bases=None, **kw):
+        from luminamoon_amd.optimizer import hip_backend
+        from oracle import oracle as O
+
+        buffer, pdt, sdt, extra = form
+        self.O, n = O, len(sizes)
+        self.group = group_dict(buffer=buffer, lr=1e-3, **{**extra, **kw})
+        self.cfg = oracle_config(O, self.group)
+        master = self.group["master_weights"] > 0
+        self.host = TensorSet(sizes, pdt, pdt, sdt, buffer in (2, "T2"), master, 83, m_scale=3e-4)
+        for v in self.host.v:
+            if v is not None:
+                v.copy_((v.float() ** 2).to(v.dtype))
+        self.offs = offs or [0] * n
+        self.ranges = ranges or [None] * n
+        self.bases = bases or [0] * n
+        self.dev, self.fill = _large(self.host)
+        for xs in (self.dev.p, self.dev.m, self.dev.v, self.dev.mp):
+            xs[:n] = [self._view(x, k) for x, k in zip(xs, self.offs)]
+        self.tables = [torch.tensor(r, dtype=torch.int64, device="cuda") if r else None for r in self.ranges] + [None]
+        self.stepper = hip_backend.HipStepper()
+
+    @staticmethod
+    def _view(x, k):
+        if x is None:
+            return None
+        big = torch.zeros(x.numel() + 256, dtype=x.dtype, device="cuda")
+        big[k:k + x.numel()] = x.to("cuda").reshape(-1)
+        return big[k:k + x.numel()]
+
+    def oracle(self, step):
+        """One step on the host; inactive ranges are stepped with a zero gradient and put back."""
+        h = self.host
+        grads = h.grads(step, 84)
+        kept = []
+        for i, rs in enumerate(self.ranges):
+            for b, e in rs or []:
+                grads[i][b:e] = 0
+                kept += [(xs[i], b, e, xs[i][b:e].clone()) for xs in (h.p, h.m, h.v, h.mp) if xs[i] is not None]
+        self.O.step(self.cfg, h.p, grads, h.m, h.v, h.mp, h.sc, [step] * len(h.sizes), list(range(len(h.sizes))), threads=4,
+                    index_bases=self.bases)
+        for x, b, e, old in kept:
+            x[b:e] = old
+        return grads
+
+    def device_grads(self, grads):
+        return [self._view(g, k) for g, k in zip(grads, self.offs)] + [self.fill]
+
+    def prepare(self, grads, step):
+        d, n = self.dev, len(self.dev.sizes)
+        return self.stepper.prepare(d.p, grads, d.m, d.v, d.mp, d.sc, [step] * n, list(range(n)), self.bases + [0], self.tables)
+
+    def steps(self, steps, label):
+        for step in steps:
+            grads = self.device_grads(self.oracle(step))  # held until the step has run
+            self.stepper.launch(self.group, self.prepare(grads, step))
+            self.check(f"{label} step {step}")
+
+    def check(self, label):
+        torch.cuda.synchronize()
+        self.host.assert_equal(self.dev, label)
+        assert int(torch.count_nonzero(self.dev.m[-1])) == 0, label  # the zero tensor stayed zero
+        assert all(int(torch.count_nonzero(ws)) == 0 for ws in self.stepper.workspace._bufs.values()), label
+
+
+def _skip_without_gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a ROCm GPU")
+
+
+@pytest.mark.parametrize("count", [len(EDGES), 60], ids=["inline", "table"])
+@pytest.mark.parametrize("form", FORMS, ids=FORM_IDS)
+def test_large_views_inactive_ranges_and_index_bases(form, count):
+    """Heads of 0 to 255 elements (views at +0 to +193, shorter tensors among them), inactive ranges over
+    heads, part and whole units and the tensor's end, shards whose offsets pass 2^31; the first step counts
+    and applies, the second is fused, the third keeps two passes."""
+    _skip_without_gpu()
+    sizes = [EDGES[i % len(EDGES)] for i in range(count)]
+    offs = [(0, 1, 33, 63, 64, 130, 193)[i % 7] for i in range(count)]
+
+    def ranges(i, n):
+        if i % 3 == 0:
+            return None
+        if i % 11 == 1:
+            return [(0, n)]
+        rs = [(0, 2), (100, 190), (255, 1300), (2048, 5120), (6000, 6001), (n - 300, n)]
+        out = []
+        for b, e in rs:
+            b, e = max(b, out[-1][1] + 1 if out else 0), min(e, n)
+            if b < e:
+                out.append((b, e))
+        return out
+
+    case = _Case(form, sizes, offs, [ranges(i, n) for i, n in enumerate(sizes)], [i * 0x13579BDF for i in range(count)])
+    print(f"[case] views and ranges {form} tensors={count}", flush=True)
+    case.steps((1, 2), f"{form}")
+    case = _Case(form, sizes, offs, case.ranges, case.bases, fused_single_pass=False)
+    case.steps((2,), f"{form} two passes")
+
+
+@pytest.mark.parametrize("count", [len(EDGES), 60], ids=["inline", "table"])
+@pytest.mark.parametrize("form", FORMS, ids=FORM_IDS)
+def test_large_single_pass_matches_oracle(form, count):
+    """cautious=False: one pass that counts nothing, with views."""
+    _skip_without_gpu()
+    case = _Case(form, [EDGES[i % len(EDGES)] for i in range(count)], [(0, 1, 130)[i % 3] for i in range(count)], cautious=False)
+    print(f"[case] single pass {form} tensors={count}", flush=True)
+    case.steps((1, 2), f"{form}")
+
+
+@pytest.mark.parametrize("count", [len(EDGES), 60], ids=["inline", "table"])
+@pytest.mark.parametrize("form", [FORMS[1], FORMS[4], FORMS[6], FORMS[10], FORMS[14]], ids=lambda f: f"{f[0]}-{f[1]}-{f[2]}")
+def test_large_launches_in_pieces_match_oracle(form, count, monkeypatch):
+    """A unit space cut into launches of 6,001 blocks: tensors straddle the cuts."""
+    _skip_without_gpu()
+    monkeypatch.setenv("LV_MAX_GRID_BLOCKS", "6001")
+    case = _Case(form, [EDGES[i % len(EDGES)] for i in range(count)], [(0, 1, 130)[i % 3] for i in range(count)])
+    print(f"[case] pieces {form} tensors={count}", flush=True)
+    case.steps((1, 2), f"{form}")
+
+
+@pytest.mark.parametrize("form", FORMS, ids=FORM_IDS)
+def test_large_graph_steps_match_oracle(form):
+    """Steps from a device record, eagerly and as replays of a captured graph, with eager work between."""
+    _skip_without_gpu()
+    case = _Case(form, EDGES, [(0, 1, 130)[i % 3] for i in range(len(EDGES))])
+    print(f"[case] graph {form}", flush=True)
+    grads = case.oracle(2)
+    static = case.device_grads(grads)
+    prep = case.prepare(static, 0)
+    rec = torch.zeros(4, dtype=torch.int64, device="cuda")
+    rec[0] = 1
+    ws = case.stepper.graph_workspace(case.group, prep)
+    case.stepper.launch_graph(case.group, prep, rec, ws)
+    case.check(f"{form} step 2")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        case.stepper.launch_graph(case.group, prep, rec, ws)
+    for step in (3, 4, 5):
+        for s, g in zip(static, case.oracle(step)):
+            s.copy_(g)
+        torch.cuda.synchronize()
+        graph.replay()
+        case.check(f"{form} replay of step {step}")
+        assert int(rec[0]) == step and int(torch.count_nonzero(ws)) == 0

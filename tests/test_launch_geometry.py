@@ -41,3 +41,20 @@ def test_every_launch_has_its_kernels_geometry(walk):
     m = re.search(r"(\d+) calls, (\d+) unit launches checked, (\d+) of large forms, (\d+) of one-wave blocks, 0 mismatches", res.stdout)
     assert m, res.stdout[-2000:]
     assert all(int(x) > 1000 for x in m.groups())  # the walk reached what it is for
+
+
+def test_gpu_tests_of_large_launches_reach_them(walk):
+    """Every form that tests/test_gpu_large_launches.py steps takes its large-launch kernel there, so those
+    tests fail to cover what they are for as soon as a rule of the dispatch moves past their sizes."""
+    from luminamoon_amd.optimizer.hip_backend import BUFFER_CODES
+    from tests.test_gpu_large_launches import EDGES, FORMS, LARGE
+
+    code = {"f32": 0, "bf16": 1, "f16": 2}
+    for buffer, pdt, sdt, extra in FORMS:
+        for count in (len(EDGES), 60):
+            sizes = [EDGES[i % len(EDGES)] for i in range(count)] + [LARGE]
+            args = [BUFFER_CODES[buffer], code[pdt], code[sdt], int("master_weights" in extra), *sizes]
+            res = subprocess.run([*walk, "route", *map(str, args)], capture_output=True, text=True, timeout=60)
+            assert res.returncode == 0, res.stdout + res.stderr
+            launches = [tuple(map(int, l.split())) for l in res.stdout.split("\n") if l]
+            assert len(launches) == 1 and launches[0][0] >> 30 == 1, (buffer, pdt, sdt, extra, count, launches)
