@@ -2036,12 +2036,13 @@ __global__ void __launch_bounds__(unit_threads(MODE, PT, ST, PASS, FL, TABLE), u
             }
         } else {
             if (!vec) cnt = wave_sum(cnt);  // block-uniform branch
-            if ((threadIdx.x & 63) == 0) sh.cnt[threadIdx.x >> 6] = cnt;
+            uint32_t *wave_cnt = reinterpret_cast<uint32_t *>(sh.cnt);
+            if ((threadIdx.x & 63) == 0) wave_cnt[threadIdx.x >> 6] = cnt;
             __syncthreads();
             if (threadIdx.x == 0) {
                 uint32_t tot = 0;
 #pragma unroll
-                for (int k = 0; k < TPB / 64; k++) tot += (uint32_t)sh.cnt[k];
+                for (int k = 0; k < TPB / 64; k++) tot += wave_cnt[k];
                 report_count<MODE, PASS, TABLE, (uint32_t)kUnit>(a, D, tv, unit, tot);
             }
         }
