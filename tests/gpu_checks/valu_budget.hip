@@ -28,4 +28,17 @@ template __global__ void unit_kernel<LV_BUFFER_DUAL, LV_DTYPE_F32, LV_DTYPE_F32,
 template __global__ void unit_kernel<LV_BUFFER_TDCLM, LV_DTYPE_F32, LV_DTYPE_F32, kFused,
                                      static_flags(LV_DTYPE_F32, kFused), true>(const Args);
 
+// The large-launch forms (kFLarge), which cfg5 and cfg3 run, and optimistic lanes in table launches: CLM with
+// bf16 params and f32 or bf16 state, TD-CLM with bf16 params and f32 state
+template __global__ void unit_kernel<LV_BUFFER_T2, LV_DTYPE_BF16, LV_DTYPE_F32, kFused,
+                                     static_flags(LV_DTYPE_BF16, kFused) | kFLarge, false>(const Args);
+template __global__ void unit_kernel<LV_BUFFER_DUAL, LV_DTYPE_F32, LV_DTYPE_F32, kFused,
+                                     static_flags(LV_DTYPE_F32, kFused) | kFLarge, false>(const Args);
+template __global__ void unit_kernel<LV_BUFFER_DUAL, LV_DTYPE_BF16, LV_DTYPE_F32, kFused,
+                                     static_flags(LV_DTYPE_BF16, kFused) | kFLarge, true>(const Args);
+template __global__ void unit_kernel<LV_BUFFER_DUAL, LV_DTYPE_BF16, LV_DTYPE_BF16, kFused,
+                                     static_flags(LV_DTYPE_BF16, kFused) | kFLarge, true>(const Args);
+template __global__ void unit_kernel<LV_BUFFER_TDCLM, LV_DTYPE_BF16, LV_DTYPE_F32, kFused,
+                                     static_flags(LV_DTYPE_BF16, kFused) | kFLarge, true>(const Args);
+
 }  // namespace lv

@@ -75,7 +75,8 @@ def issue_units(op: str) -> float:
 #   T2: clm / env, the coordinate bound's quotient; sqrt(v). T1: the same without v.
 #   CLM: clm / sigma, the bound's step / b, two tanh quotients; sqrt(v), sqrt(p^2 + 1e-4).
 #   TD-CLM: clm / env, step / b, one tanh quotient; sqrt(p^2 + 1e-4).
-#   fp16 params add the fp16 safety bound's quotient.
+#   fp16 params add the fp16 safety bound's quotient. Lanes add one reciprocal a lane (lane_min_u).
+# "large" are the forms of launches of 2^25 elements or more, which cfg3 and cfg5 run.
 IEEE2 = {"v_rcp_f32": 2, "v_div_fixup_f32": 2}
 FAST2 = {"v_rcp_f32": 2, "v_div_fixup_f32": 0}
 KERNELS = {
@@ -94,6 +95,16 @@ KERNELS = {
                      {"v_rcp_f32": 4, "v_div_fixup_f32": 4, "v_rsq_f32": 2, "v_mul_lo_u32": 0}),
     "cfg2 TD-CLM f32, table": ("_ZN2lv11unit_kernelILi1ELi0ELi0ELi1ELj75ELb1EEEvNS_4ArgsE", 4, 96.5,
                                {"v_rcp_f32": 3, "v_div_fixup_f32": 3, "v_rsq_f32": 1, "v_mul_lo_u32": 0}),
+    "cfg5 T2 bf16, f32 m/v, large": ("_ZN2lv11unit_kernelILi4ELi1ELi0ELi1ELj1073742155ELb0EEEvNS_4ArgsE", 4, 91.5,
+                                     {**IEEE2, "v_rsq_f32": 1, "v_mul_lo_u32": 2, "v_cvt_sr_bf16_f32": 0}),
+    "cfg3 CLM f32, large": ("_ZN2lv11unit_kernelILi2ELi0ELi0ELi1ELj1073741899ELb0EEEvNS_4ArgsE", 4, 142.0,
+                                  {"v_rcp_f32": 4, "v_div_fixup_f32": 4, "v_rsq_f32": 2, "v_mul_lo_u32": 0}),
+    "CLM bf16, f32 m/v, lanes": ("_ZN2lv11unit_kernelILi2ELi1ELi0ELi1ELj1073742155ELb1EEEvNS_4ArgsE", 4, 123.5,
+                                 {"v_rcp_f32": 4.25, "v_div_fixup_f32": 0, "v_rsq_f32": 2, "v_mul_lo_u32": 2}),
+    "CLM bf16, bf16 m/v, lanes": ("_ZN2lv11unit_kernelILi2ELi1ELi1ELi1ELj1073742155ELb1EEEvNS_4ArgsE", 8, 140.0,
+                                  {"v_rcp_f32": 4.125, "v_div_fixup_f32": 0, "v_rsq_f32": 2, "v_mul_lo_u32": 6}),
+    "TD-CLM bf16, f32 m, lanes": ("_ZN2lv11unit_kernelILi1ELi1ELi0ELi1ELj1073742155ELb1EEEvNS_4ArgsE", 4, 90.5,
+                                  {"v_rcp_f32": 3.25, "v_div_fixup_f32": 0, "v_rsq_f32": 1, "v_mul_lo_u32": 2}),
 }
 
 CATEGORIES = [
