@@ -731,7 +731,7 @@ static void fill_desc(Desc &D, const lv_tensor &T, const Item &it, bool dual, ui
     D.scratch = T.scratch;
     D.n = T.numel;
     D.unit_begin = 0;
-    D.pidx = (uint32_t)T.param_index;
+    D.pidx = (uint32_t)T.param_index & 0x7FFFFFFFu;
     D.ibase = (uint32_t)T.index_base;
     D.nskip = (uint32_t)T.n_inactive;  // < 2^24 (prepare_call)
     uint32_t head = 0;

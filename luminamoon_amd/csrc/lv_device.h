@@ -243,15 +243,15 @@ struct Desc {
     void *v;
     float *mp;
     float *scratch;
-    uint64_t n : 63;    // elements (at most 2^40)
+    uint64_t n;
+    uint32_t unit_begin;  // first work unit of this tensor in the launch's unit space
+    uint32_t pidx : 31;   // low bits of param_index (seeds only need idx * 10007 mod 2^31)
     // vec: every stream is aligned at element `head` (one-wave kernels: at most 255 elements, to whole
     // 256-element pieces of every stream where the views allow it; others: at most 63, to a 128-byte line;
     // else to 16 bytes), so the tensor's work units start there and whole units take the vector path; the
     // `head` elements before it are taken by one block (unit_kernel's takes_head). Set by the host from
     // the pointers.
-    uint64_t vec : 1;
-    uint32_t unit_begin;  // first work unit of this tensor in the launch's unit space
-    uint32_t pidx;        // low 32 bits of param_index (seeds only need idx * 10007 mod 2^31)
+    uint32_t vec : 1;
     uint32_t ibase;       // low 32 bits of index_base (the SR offset is taken mod 2^32)
     uint32_t nskip : 24;  // inactive [begin, end) ranges in `skip` (sorted, disjoint)
     uint32_t head : 8;
