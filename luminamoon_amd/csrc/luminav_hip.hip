@@ -820,7 +820,7 @@ static PassPlan plan_pass(const lv_config *cfg, const Args &args, const Item &h,
     const bool large = elems >= kLargeElems &&
                        (!unit_lanes(cfg->buffer, h.pt, h.st, pass, p.flags | kFLarge) || lane_facts(cfg, args));
     p.kernel = pick_kernel(cfg->buffer, h.pt, h.st, pass, large ? p.flags | kFLarge : p.flags, table);
-    if (table && p.kernel.threads < kThreads && elems < (uint64_t)count * wave_table_mean(cfg->buffer, h.pt, h.master))
+    if (table && p.kernel.threads < kThreads && elems < (uint64_t)count * wave_table_mean(cfg->buffer, h.pt, pass, h.master))
         p.kernel = pick_kernel(cfg->buffer, h.pt, h.st, pass, p.flags, table);
     return p;
 }

@@ -127,7 +127,7 @@ constexpr int unit_min_blocks(int mode, int pt, int st, int pass, uint32_t flags
     return unit_subs(mode, pt, st, pass, flags) > 1 && pass != kCount ? 8 : 1;
 }
 
-// Resident one-wave blocks per CU of a large f32-state launch, 0 where it keeps 256-thread blocks.
+// Resident one-wave blocks per CU of a large f32-state launch.
 //
 // The f32-state steps are bound by HBM, and HBM's rate depends on how many waves stream at once. A
 // full CU (32 waves) puts more requests in flight than the memory system keeps in order, and the
@@ -153,8 +153,8 @@ constexpr int unit_min_blocks(int mode, int pt, int st, int pass, uint32_t flags
 //   T2   f16 + master, table        4600.4    32: 4430.2  18: 4270.8  16: 4148.9  14: 4197.2
 //
 // More arithmetic per byte needs more waves, more bytes per wave fewer. T1 with 16-bit params and no
-// master moves too few bytes per wave for a limit and keeps 256-thread blocks: one-wave table launches
-// of 100 tensors ran 0.75-0.98x at 1.7e7-6e8 elements, inline ones level. CLM and TD-CLM with 16-bit params and no
+// master moves too few bytes per wave for a limit, and its fused step keeps 256-thread blocks (unit_large).
+// CLM and TD-CLM with 16-bit params and no
 // master are bound by their arithmetic, and one-wave blocks alone change nothing there (CLM f16 4143 ->
 // 4167, TD bf16 2336 -> 2331); with optimistic lanes (unit_lanes): CLM bf16 32: 3511.9  25: 3459.5  21:
 // 3387.9, CLM f16 32: 3826.3  25: 3847.3, TD bf16 32: 2125.4  25: 2255.9, TD f16 32: 2802.1  25: 2832.7.
@@ -164,29 +164,33 @@ constexpr uint32_t wave_resident(int mode, int pt, bool master) {
     if (master) return mode == LV_BUFFER_TDCLM ? 25u : mode == LV_BUFFER_DUAL ? 21u : mode == LV_BUFFER_T1 ? 18u : 16u;
     if (mode == LV_BUFFER_T2) return pt == LV_DTYPE_BF16 ? 18u : 25u;
     if (mode == LV_BUFFER_DUAL && pt == LV_DTYPE_BF16) return 21u;
-    return mode == LV_BUFFER_T1 ? 0u : 32u;
+    return 32u;
 }
 
-// Whether the large form of a table launch runs one-wave blocks too. A table launch has the count slots
-// of 1024-element units (the workspace is sized for those), so up to 256 one-wave blocks report to one
-// slot, and atomics of several XCDs on one line take turns: 50-500 tensors of 1.3e6 elements or less ran
-// 0.75-1.0x of 256-thread blocks, with 64 blocks per slot 0.93-1.07x, without reports 0.97-1.08x (four
-// slots to a line are as slow as one). One-wave blocks pay for that only where a limit on them gains
-// more: not at 32 per CU, where 256-thread blocks of the same lanes are as fast (f32 state, 60 and 400
-// tensors and two models, 3.4e7-9.5e8 elements, against the general path: TD bf16 1.06-1.09x, TD f16
-// 1.05-1.10x, CLM f16 1.03-1.06x), nor for TD-CLM with a master (1.06-1.11x, one-wave 1.05-1.14x).
-constexpr bool wave_table(int mode, int pt, bool master) {
-    return wave_resident(mode, pt, master) < 32u && !(mode == LV_BUFFER_TDCLM && master);
+// Whether the large form of a table launch runs one-wave blocks too. The applying and single passes do; a
+// fused pass also reports its counts. A table launch has the count slots of 1024-element units (the
+// workspace is sized for those), so up to 256 one-wave blocks report to one slot, and atomics of several
+// XCDs on one line take turns: 50-500 tensors of 1.3e6 elements or less ran 0.75-1.0x of 256-thread blocks,
+// with 64 blocks per slot 0.93-1.07x, without reports 0.95-1.08x (four slots to a line are as slow as
+// one). Fused one-wave blocks pay for that only where a limit on them gains more: not at 32 per CU, where
+// 256-thread blocks of the same lanes are as fast (f32 state, 60 and 400 tensors and two models,
+// 3.4e7-9.5e8 elements, against the general path: TD bf16 1.06-1.09x, TD f16 1.05-1.10x, CLM f16
+// 1.03-1.06x), nor for TD-CLM with a master (1.06-1.11x, one-wave 1.05-1.14x).
+constexpr bool wave_table(int mode, int pt, int pass, bool master) {
+    return pass != kFused || (wave_resident(mode, pt, master) < 32u && !(mode == LV_BUFFER_TDCLM && master));
 }
 
 // Smallest mean tensor of a one-wave table launch, in elements: larger tensors have the most count slots
-// either way, and finish a slot's blocks over a longer time. Against 256-thread blocks, ragged lists of
-// 60-400 tensors and GPT-2 and Llama shapes, by mean tensor:
+// either way, and finish a slot's blocks over a longer time. Fused steps against 256-thread blocks, ragged
+// lists of 60-400 tensors and GPT-2 and Llama shapes, by mean tensor:
 //   28 bytes an element (CLM, T2: f32, or with a master)   0.35-0.9e6: 0.93-1.08x   1.1e6 and up: 1.00-1.13x
 //   20-22 bytes                                             0.35-0.9e6: 0.80-1.08x   1.1-1.9e6: 0.94-1.09x
 //                                                           2.2e6 and up: 0.96-1.06x (means 1.01-1.05x)
-constexpr uint64_t wave_table_mean(int mode, int pt, bool master) {
+// The passes without reports (500 tensors): T1 f32 0.93x at 3e4, 0.97x at 9e4, 1.00x at 2.6e5, CLM f32 1.01x,
+// 1.06x, 1.12x.
+constexpr uint64_t wave_table_mean(int mode, int pt, int pass, bool master) {
     const bool two = mode == LV_BUFFER_DUAL || mode == LV_BUFFER_T2;
+    if (pass != kFused) return two ? 0 : 1ull << 18;
     return two && (pt == LV_DTYPE_F32 || master) ? 1ull << 20 : 1ull << 21;
 }
 
@@ -210,7 +214,9 @@ constexpr bool unit_large(int mode, int pt, int st, int pass, uint32_t flags) {
     if (pt == LV_DTYPE_F32 && (flags & kFMaster)) return false;
     const bool arithmetic = (mode == LV_BUFFER_DUAL || mode == LV_BUFFER_TDCLM) && pt != LV_DTYPE_F32 && !(flags & kFMaster);
     if (st != LV_DTYPE_F32 || arithmetic) return unit_lanes(mode, pt, st, pass, flags | kFLarge);
-    return wave_resident(mode, pt, (flags & kFMaster) != 0) != 0;
+    // T1 with 16-bit params and no master: fused one-wave table launches of 100 tensors ran 0.75-0.98x at
+    // 1.7e7-6e8 elements, without reports 1.00-1.06x; fused inline launches level
+    return !(mode == LV_BUFFER_T1 && pt != LV_DTYPE_F32 && !(flags & kFMaster) && pass == kFused);
 }
 
 // Threads per block of the unit kernel for this mode, dtypes, pass, flag word (the launch's word;
@@ -221,7 +227,7 @@ constexpr bool unit_large(int mode, int pt, int st, int pass, uint32_t flags) {
 // - T2 with bf16 params (the headline's kernel): 0.966x at 1e9 elements, 0.959x at 3.5e9.
 constexpr int unit_threads(int mode, int pt, int st, int pass, uint32_t flags, bool table) {
     if (flags & kFLarge)
-        return pass == kCount || st != LV_DTYPE_F32 || (table && !wave_table(mode, pt, (flags & kFMaster) != 0)) ? kThreads : 64;
+        return pass == kCount || st != LV_DTYPE_F32 || (table && !wave_table(mode, pt, pass, (flags & kFMaster) != 0)) ? kThreads : 64;
     const bool one_wave = (mode == LV_BUFFER_DUAL && pt == LV_DTYPE_F32) || (mode == LV_BUFFER_T2 && pt == LV_DTYPE_BF16);
     return (!table && one_wave && st == LV_DTYPE_F32 && pass == kFused && flags == static_flags(pt, pass)) ? 64 : kThreads;
 }

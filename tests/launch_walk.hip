@@ -250,7 +250,7 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
         const uint32_t wanted = base & lv::kFDynamic ? a.flags : base;  // a dynamic kernel may stand in for a large form
         bool take = lv::unit_large(k.mode, k.pt, k.st, k.pass, wanted) && elems >= lv::kLargeElems;
         if (k.table && lv::unit_threads(k.mode, k.pt, k.st, k.pass, wanted | lv::kFLarge, true) == 64)
-            take = take && elems >= (uint64_t)a.ndesc * lv::wave_table_mean(k.mode, k.pt, master);
+            take = take && elems >= (uint64_t)a.ndesc * lv::wave_table_mean(k.mode, k.pt, k.pass, master);
         // lanes take no launch whose steps would mostly fall below their range
         if (lanes) take = take && c.lr >= 0x1p-30f;
         const bool large = (k.fl & lv::kFLarge) != 0;
@@ -325,6 +325,7 @@ int main(int argc, char **argv) {
         {"inline large", 5, (1u << 25) + 7, nullptr},
         {"table large", 60, (1u << 27) + 7, nullptr},
         {"table of small tensors", 60, (1u << 25) + 7, nullptr},
+        {"table of many small tensors", 150, (1u << 25) + 7, nullptr},
         {"table split", 60, 0, "50"},
     };
     static const uint64_t sizes[] = {1, 300, 1025, 4097, 70001, 64 * 1024 + 1};
@@ -345,7 +346,7 @@ int main(int argc, char **argv) {
                 T.push_back(tensor(i, n, pt, gt, st, dual, master, offs[i % 5], goffs[i % 5]));
             }
             for (float lr : {1e-3f, 9.5e-10f, 9e-10f, 0.0f})
-            for (int opt = lr == 1e-3f ? 0 : 7; opt < 8; opt++)
+            for (int opt = lr == 1e-3f && sh.count < 100 ? 0 : 6; opt < 8; opt++)
             for (int bound = 0; bound < 3; bound++)
             for (int when = 0; when < 3; when++)
             for (int entry = 0; entry < 3; entry++) {
