@@ -92,8 +92,8 @@ constexpr uint32_t static_flags(int PT, int PASS) {
 //   TD   bf16, bf16 state 2116.7 -> 1990.0       TD  bf16, f32 state 2308.4 -> 2128.1
 //   CLM  f16,  f32 state  4123.3 -> 3826.3       TD  f16,  f32 state 3079.7 -> 2807.7
 // and the same with 5% of the gradients zero for thousands of steps (m and v decayed away there): 3238.4
-// -> 2872.8 and 3726.8 -> 3422.1. T1 and T2 with 16-bit state measured 0.97-0.99x (their general path has
-// one guarded quotient less and no tanh), CLM f16 with 16-bit state 0.79x (it spills).
+// -> 2872.8 and 3726.8 -> 3422.1. T1 and T2 with 16-bit state ran at 0.97-0.99 of the general path's speed
+// (that path has one guarded quotient less there and no tanh), CLM f16 with 16-bit state at 0.79 (it spills).
 constexpr bool unit_lanes(int mode, int pt, int st, int pass, uint32_t flags) {
     const uint32_t need = (uint32_t)kFLarge | (uint32_t)kFCautious | (uint32_t)kFSR | (uint32_t)kFWeightDecay | (uint32_t)kFCoordinate;
     return pass != kCount && (flags & (need | (uint32_t)kFRadial | (uint32_t)kFMaster)) == need &&
@@ -113,7 +113,8 @@ constexpr int kLaneGroup = 2;  // elements of a lane whose arithmetic is interle
 // element, and a block of 1024 elements is mostly its own prologue: with 4096-element units, all their
 // loads in flight at once, the two passes of a 9.5e8-element bf16 step run 3450 -> 3071 us (TD-CLM)
 // and 5249 -> 4972 us (CLM), of a 1.2e8-element f32 step 821 -> 774 us (CLM); 2048-element units 3089,
-// 5060 and 774. Small launches lose (3.5e6 elements 22.1 -> 23.5 us) and keep 1024 or 2048.
+// 5060 and 774. Small launches lose (3.5e6 elements 22.1 -> 23.5 us)
+// and count in the applying pass's units.
 constexpr int unit_subs(int mode, int pt, int st, int pass, uint32_t flags) {
     if (pass == kCount && (flags & kFLarge)) return 4 / unit_halves(mode, pt, st);
     return (mode == LV_BUFFER_T1 && st != LV_DTYPE_F32 && pt != LV_DTYPE_F32 && flags == static_flags(pt, pass)) ? 2 : 1;
@@ -154,10 +155,17 @@ constexpr int unit_min_blocks(int mode, int pt, int st, int pass, uint32_t flags
 //
 // More arithmetic per byte needs more waves, more bytes per wave fewer. T1 with 16-bit params and no
 // master moves too few bytes per wave for a limit, and its fused step keeps 256-thread blocks (unit_large).
-// CLM and TD-CLM with 16-bit params and no
-// master are bound by their arithmetic, and one-wave blocks alone change nothing there (CLM f16 4143 ->
-// 4167, TD bf16 2336 -> 2331); with optimistic lanes (unit_lanes): CLM bf16 32: 3511.9  25: 3459.5  21:
-// 3387.9, CLM f16 32: 3826.3  25: 3847.3, TD bf16 32: 2125.4  25: 2255.9, TD f16 32: 2802.1  25: 2832.7.
+// CLM and TD-CLM with 16-bit params and no master are bound by their arithmetic, and one-wave blocks alone
+// change nothing there (CLM f16 4143 -> 4167, TD bf16 2336 -> 2331); with optimistic lanes (unit_lanes): CLM
+// bf16 32: 3511.9  25: 3459.5  21: 3387.9, CLM f16 32: 3826.3  25: 3847.3, TD bf16 32: 2125.4  25: 2255.9, TD
+// f16 32: 2802.1  25: 2832.7.
+//
+// At other sizes (ragged lists of 8, 45 and 60 tensors and buckets, 3.5e7-7e8 elements, 32 to 12 per CU in one
+// process) the numbers below were within 1.5% of the best, but for these. T2 in f32 or with a master ran
+// up to 3% faster at 14 from 7e7 elements on, and up to 3.5% slower at 14 in table launches of 3.5e7 or less:
+// 16. T1 in f32 or with a master ran up to 2.5% faster at 16 in buckets, and up to 4% slower in inline and
+// table launches of 7e8 or less: 18. CLM bf16 with lanes ran 1-4% faster at 25 in inline launches and buckets
+// and 1% slower in table launches: 21.
 constexpr uint32_t wave_resident(int mode, int pt, bool master) {
     if (pt == LV_DTYPE_F32)
         return mode == LV_BUFFER_T2 ? 16u : mode == LV_BUFFER_TDCLM ? 21u : 18u;
@@ -221,8 +229,8 @@ constexpr bool unit_large(int mode, int pt, int st, int pass, uint32_t flags) {
 
 // Threads per block of the unit kernel for this mode, dtypes, pass, flag word (the launch's word;
 // the run-time-flag kernels have 256) and launch kind. The kFLarge kernels that write f32 state run
-// one-wave blocks (units of 256 elements; in table launches where wave_table says so), and so do two steady inline steps with f32 state and the reference defaults at
-// every size. In one process on the same buffers, against 256-thread blocks:
+// one-wave blocks (units of 256 elements; in table launches where wave_table says so), and so do two
+// steady inline steps with f32 state and the reference defaults at every size. In one process on the same buffers, against 256-thread blocks:
 // - CLM in f32 (cfg3's kernel): 0.938-0.966x (cfg3, and a 1e9-element bucket);
 // - T2 with bf16 params (the headline's kernel): 0.966x at 1e9 elements, 0.959x at 3.5e9.
 constexpr int unit_threads(int mode, int pt, int st, int pass, uint32_t flags, bool table) {
@@ -1216,7 +1224,7 @@ __device__ __forceinline__ void lane_hi(LaneRange &r, float x) {
 // the wave (lane_ok); the launch has checked lane_facts. cs: the cautious scale; min_u: lane_min_u.
 //
 // Why the result is apply_elem's when r passes. No value in r.hi is NaN, so g, m, v' and p are not.
-// - sanitize and clamp_defect are the identity. CLM: |g|, |g - m'| <= 2^25. TD-CLM: r.den bounds the
+// - sanitize and clamp_defect are the identity. CLM: |g|, |g - m'| <= 2^25. TD-CLM: r.hi bounds the
 //   envelope, at least (1 - b1^2) |g| and b1^2 |m| with both factors >= 2^-20, so |g|, |m| <= 2^45.
 // - an element with g = 0 is masked: u * g is not above 0 whatever u is (NaN included), its step is 0,
 //   and m', v' do not depend on u. Otherwise:
@@ -1803,10 +1811,9 @@ __device__ __forceinline__ int find_tensor(const Args &a, uint32_t unit) {
 // completion in ONE 64-bit atomic (count << kTicketBits | 1) on one of the tensor's S count slots
 // (slot = unit index in the tensor mod S, 64 B apart, so the atomics spread over L2 channels;
 // S = launch_count_slots: the smallest power of two keeping every slot at <= 64 blocks (256 one-wave
-// blocks of a table launch), at
-// most 64). The block whose report completes a slot (its ticket reaches the slot's block count)
+// blocks of a table launch), at most 64). The block whose report completes a slot (its ticket reaches the slot's block count)
 // holds that slot's whole count in the value its own atomic returned and re-zeroes the slot; a
-// tensor of one slot (<= 64 units) is then complete, and that block finalises the scratch. With
+// tensor of one slot (at most that many units) is then complete, and that block finalises the scratch. With
 // more slots it reports count << kFoldBits | 1 on the tensor's fold slot (the one after its count
 // slots), and the block that completes the fold slot holds the tensor's exact count and
 // finalises the scratch. Every decision reads only the value
@@ -1831,7 +1838,7 @@ __device__ __forceinline__ void report_count(const Args &a, const Desc &D, const
     if ((uint32_t)(old & kTicketMask) + 1u != expect) return;
     const unsigned long long slot_count = (old >> kTicketBits) + count;
     __hip_atomic_store(slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (nslots == 1u) {  // a tensor of <= 64 units: its one slot holds its whole count
+    if (nslots == 1u) {  // the tensor's one slot holds its whole count
         finalize_scratch<MODE, PASS>(a, false, D, slot_count, 0.0f, 0.0f);
         return;
     }
