@@ -125,7 +125,7 @@ constexpr int unit_subs(int mode, int pt, int st, int pass, uint32_t flags) {
 // the bound keeps 8 and 78 SGPRs): 1.635 against 1.612 ms for bf16-state cfg4.
 constexpr int unit_min_blocks(int mode, int pt, int st, int pass, uint32_t flags) {
     if (unit_lanes(mode, pt, st, pass, flags)) return st != LV_DTYPE_F32 ? 8 : 1;
-    return unit_subs(mode, pt, st, pass, flags) > 1 && pass != kCount ? 8 : 1;
+    return unit_subs(mode, pt, st, pass, flags) > 1 && !(pass == kCount && (flags & kFLarge)) ? 8 : 1;
 }
 
 // Resident one-wave blocks per CU of a large f32-state launch.
