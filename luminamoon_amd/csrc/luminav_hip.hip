@@ -732,13 +732,13 @@ static void fill_desc(Desc &D, const lv_tensor &T, const Item &it, bool dual, ui
     D.scratch = T.scratch;
     D.n = T.numel;
     D.unit_begin = 0;
-    D.pidx = (uint32_t)T.param_index & 0x7FFFFFFFu;
+    D.pidx = (uint32_t)T.param_index;
     D.ibase = (uint32_t)T.index_base;
     D.nskip = (uint32_t)T.n_inactive;  // < 2^24 (prepare_call)
     uint32_t head = 0;
     D.vec = vector_head(T, it, dual, unit_elems, head) ? 1u : 0u;
     D.head = head;
-    D.skip = T.n_inactive ? T.inactive : nullptr;
+    D.skip_addr = T.n_inactive ? (uint64_t)(uintptr_t)T.inactive : 0;
 }
 
 // Work units of a tensor: they start at its vector head, so an unaligned view may have one fewer

@@ -259,17 +259,20 @@ struct Desc {
     float *scratch;
     uint64_t n;
     uint32_t unit_begin;  // first work unit of this tensor in the launch's unit space
-    uint32_t pidx : 31;   // low bits of param_index (seeds only need idx * 10007 mod 2^31)
+    uint32_t pidx;        // low 32 bits of param_index (seeds only need idx * 10007 mod 2^31)
+    uint32_t ibase;       // low 32 bits of index_base (the SR offset is taken mod 2^32)
+    uint32_t nskip : 24;  // inactive [begin, end) ranges at skip() (sorted, disjoint)
+    uint32_t head : 8;
+    uint64_t skip_addr : 63;
     // vec: every stream is aligned at element `head` (one-wave kernels: at most 255 elements, to whole
     // 256-element pieces of every stream where the views allow it; others: at most 63, to a 128-byte line;
     // else to 16 bytes), so the tensor's work units start there and whole units take the vector path; the
     // `head` elements before it are taken by one block (unit_kernel's takes_head). Set by the host from
-    // the pointers.
-    uint32_t vec : 1;
-    uint32_t ibase;       // low 32 bits of index_base (the SR offset is taken mod 2^32)
-    uint32_t nskip : 24;  // inactive [begin, end) ranges in `skip` (sorted, disjoint)
-    uint32_t head : 8;
-    const uint64_t *skip;
+    // the pointers. It shares a word with the rarely read address: beside the element count its mask took
+    // scalar registers some kernels spilled (T1 with bf16 state, table launch: 68 -> 300 lane reads), beside
+    // pidx it drew that load into the prologue (T1 f16 with f32 state, 3.5e7 elements 85.6 -> 89.5 us).
+    uint64_t vec : 1;
+    __host__ __device__ const uint64_t *skip() const { return reinterpret_cast<const uint64_t *>((uintptr_t)skip_addr); }
 };
 
 // A tensor of a table launch, in device memory: its descriptor, the end of its unit range and the
@@ -1474,7 +1477,7 @@ __device__ __forceinline__ Desc table_desc(const Args &a, int t) {
     d.nskip = c.nskip;
     d.head = c.head;
     d.vec = c.vec;
-    d.skip = c.skip;
+    d.skip_addr = c.skip_addr;
     return d;
 }
 
@@ -1721,8 +1724,8 @@ __device__ __forceinline__ void scalar_range(const Args &a, const Desc &D, const
     for (uint64_t i = e_begin; i < e_end; i++) {
         bool inactive = false;
         if (nskip) {
-            while (r < nskip && ((const LV_GLOBAL uint64_t *)D.skip)[2 * r + 1] <= i) r++;
-            inactive = r < nskip && ((const LV_GLOBAL uint64_t *)D.skip)[2 * r] <= i;
+            while (r < nskip && ((const LV_GLOBAL uint64_t *)D.skip())[2 * r + 1] <= i) r++;
+            inactive = r < nskip && ((const LV_GLOBAL uint64_t *)D.skip())[2 * r] <= i;
         }
         float g = inactive ? 0.0f : load1_dyn(gdt, D.g, i);
         float m = load1<ST>(D.m, i);
@@ -1761,12 +1764,12 @@ __device__ __forceinline__ int inactive_cover(const Desc &D, uint64_t e0, uint64
     uint32_t lo = 0, hi = D.nskip;
     while (lo < hi) {
         uint32_t mid = (lo + hi) >> 1;
-        if (((const LV_GLOBAL uint64_t *)D.skip)[2 * mid + 1] <= e0) lo = mid + 1;
+        if (((const LV_GLOBAL uint64_t *)D.skip())[2 * mid + 1] <= e0) lo = mid + 1;
         else hi = mid;
     }
     first = lo;
     if (lo == D.nskip) return 0;
-    const uint64_t b = ((const LV_GLOBAL uint64_t *)D.skip)[2 * lo], e = ((const LV_GLOBAL uint64_t *)D.skip)[2 * lo + 1];
+    const uint64_t b = ((const LV_GLOBAL uint64_t *)D.skip())[2 * lo], e = ((const LV_GLOBAL uint64_t *)D.skip())[2 * lo + 1];
     if (b >= e1) return 0;
     return (b <= e0 && e >= e1) ? 2 : 1;
 }
