@@ -737,14 +737,15 @@ static void fill_desc(Desc &D, const lv_tensor &T, const Item &it, bool dual, ui
     D.nskip = (uint32_t)T.n_inactive;  // < 2^24 (prepare_call)
     uint32_t head = 0;
     D.vec = vector_head(T, it, dual, unit_elems, head) ? 1u : 0u;
-    D.head = head;
+    D.head_lo = head & 63u;
+    D.head_hi = head >> 6;
     D.skip_addr = T.n_inactive ? (uint64_t)(uintptr_t)T.inactive : 0;
 }
 
 // Work units of a tensor: they start at its vector head, so an unaligned view may have one fewer
 // than an aligned tensor of the same size (never more: call_needs counts from element 0).
 static uint64_t desc_units(const Desc &D, uint32_t unit_elems) {
-    return units_of(D.n - (D.vec ? D.head : 0u), unit_elems);
+    return units_of(D.n - (D.vec ? D.head() : 0u), unit_elems);
 }
 
 // The facts about the hyper-parameters that optimistic lanes (lane_update) rely on. They hold for

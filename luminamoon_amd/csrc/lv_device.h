@@ -194,11 +194,11 @@ constexpr bool wave_table(int mode, int pt, int pass, bool master) {
 //   28 bytes an element (CLM, T2: f32, or with a master)   0.35-0.9e6: 0.93-1.08x   1.1e6 and up: 1.00-1.13x
 //   20-22 bytes                                             0.35-0.9e6: 0.80-1.08x   1.1-1.9e6: 0.94-1.09x
 //                                                           2.2e6 and up: 0.96-1.06x (means 1.01-1.05x)
-// The passes without reports (500 tensors): T1 f32 0.93x at 3e4, 0.97x at 9e4, 1.00x at 2.6e5, CLM f32 1.01x,
-// 1.06x, 1.12x.
+// The passes without reports: T1 f32 (500 tensors) 0.93x at 3e4, 0.97x at 9e4, 1.00x at 2.6e5; CLM f32 1.01x,
+// 1.06x, 1.12x; the steps with 16-bit params 1.02-1.09x at 1e5 (400 tensors, two passes).
 constexpr uint64_t wave_table_mean(int mode, int pt, int pass, bool master) {
     const bool two = mode == LV_BUFFER_DUAL || mode == LV_BUFFER_T2;
-    if (pass != kFused) return two ? 0 : 1ull << 18;
+    if (pass != kFused) return mode == LV_BUFFER_T1 && pt == LV_DTYPE_F32 ? 1ull << 18 : 0;
     return two && (pt == LV_DTYPE_F32 || master) ? 1ull << 20 : 1ull << 21;
 }
 
@@ -262,16 +262,20 @@ struct Desc {
     uint32_t pidx;        // low 32 bits of param_index (seeds only need idx * 10007 mod 2^31)
     uint32_t ibase;       // low 32 bits of index_base (the SR offset is taken mod 2^32)
     uint32_t nskip : 24;  // inactive [begin, end) ranges at skip() (sorted, disjoint)
-    uint32_t head : 8;
-    uint64_t skip_addr : 63;
-    // vec: every stream is aligned at element `head` (one-wave kernels: at most 255 elements, to whole
+    // vec: every stream is aligned at element head() (one-wave kernels: at most 255 elements, to whole
     // 256-element pieces of every stream where the views allow it; others: at most 63, to a 128-byte line;
     // else to 16 bytes), so the tensor's work units start there and whole units take the vector path; the
-    // `head` elements before it are taken by one block (unit_kernel's takes_head). Set by the host from
-    // the pointers. It shares a word with the rarely read address: beside the element count its mask took
-    // scalar registers some kernels spilled (T1 with bf16 state, table launch: 68 -> 300 lane reads), beside
-    // pidx it drew that load into the prologue (T1 f16 with f32 state, 3.5e7 elements 85.6 -> 89.5 us).
-    uint64_t vec : 1;
+    // head() elements before it are taken by one block (unit_kernel's takes_head). Set by the host from
+    // the pointers. Only one-wave kernels read the head's two high bits (open_view): with an 8-bit head
+    // beside nskip and vec in the count's, the index's or the address's word, other kernels lost by scalar
+    // loads and masks in their prologues (CLM lanes with bf16 state 0.8%, T1 f16 with f32 state 4%, TD-CLM in two
+    // passes 1.6%, each by another of the three).
+    uint32_t head_lo : 6;
+    uint32_t vec : 1;
+    uint32_t : 1;
+    uint64_t skip_addr : 62;
+    uint64_t head_hi : 2;
+    __host__ __device__ uint32_t head() const { return (uint32_t)head_hi << 6 | head_lo; }
     __host__ __device__ const uint64_t *skip() const { return reinterpret_cast<const uint64_t *>((uintptr_t)skip_addr); }
 };
 
@@ -346,7 +350,7 @@ struct Args {
 constexpr int kTableHeads = kMaxDesc * (int)(sizeof(Desc) / sizeof(uint32_t));  // 960
 
 static_assert(sizeof(Desc) == 80, "descriptor layout");
-static_assert(kMinUnitElems - 1 < (1u << 8), "heads of one-wave kernels fit Desc::head");
+static_assert(kMinUnitElems - 1 < (1u << 8), "heads of one-wave kernels fit Desc's 8 bits");
 static_assert(sizeof(TDesc) == 88, "table descriptor layout");
 static_assert(sizeof(Args) <= 4096, "kernel arguments must fit in 4 KiB");
 
@@ -1475,7 +1479,8 @@ __device__ __forceinline__ Desc table_desc(const Args &a, int t) {
     d.pidx = c.pidx;
     d.ibase = c.ibase;
     d.nskip = c.nskip;
-    d.head = c.head;
+    d.head_lo = c.head_lo;
+    d.head_hi = c.head_hi;
     d.vec = c.vec;
     d.skip_addr = c.skip_addr;
     return d;
@@ -1499,12 +1504,13 @@ struct View {
 // launches everything else a block reads before its arithmetic (open_step) waits until its stream
 // loads are in flight: each dependent scalar load before the first vector load delays every
 // block's loads by a scalar-cache round trip, and a block lives only a few microseconds.
+template <int TPB>
 __device__ __forceinline__ View open_view(const Desc &D) {
     View tv;
     tv.t_begin = D.unit_begin;
     tv.n = D.n;
     tv.vec_ok = D.vec;
-    tv.head = D.vec ? D.head : 0u;
+    tv.head = D.vec ? (TPB == kThreads ? D.head_lo : D.head()) : 0u;  // 256-thread launches: below 64
     return tv;
 }
 
@@ -1942,7 +1948,7 @@ __global__ void __launch_bounds__(unit_threads(MODE, PT, ST, PASS, FL, TABLE), u
     Desc table_d;
     if constexpr (TABLE) table_d = table_desc(a, t);
     const Desc &D = TABLE ? table_d : a.d[t];
-    View tv = open_view(D);
+    View tv = open_view<TPB>(D);
     // Table launches (many small tensors, latency-bound, descriptors in device memory) read the
     // rest of the view first: issued behind the stream loads, those reads queue after them
     // (cfg2's 64-tensor launch: 20.6 vs 18.7 us). Inline launches stream and read it afterwards.

@@ -201,7 +201,8 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
                              "kernel of other dtypes", &l);
             // whole units from the head on, every stream aligned there
             if (D.vec) {
-                const uintptr_t h = D.head;
+                const uintptr_t h = D.head();
+                ok = ok && check(threads == 64 || h < 64, "a 256-thread kernel reads six bits of the head", &l);
                 bool al = ((uintptr_t)D.p + h * bytes_of(t.param_dtype)) % 16 == 0 || bytes_of(t.param_dtype) == 2;
                 al = al && ((uintptr_t)D.p + h * bytes_of(t.param_dtype)) % 16 == 0;
                 al = al && ((uintptr_t)D.g + h * bytes_of(t.grad_dtype)) % 16 == 0;
@@ -217,7 +218,7 @@ static void check_call(const lv_config &c, std::vector<lv_tensor> &T, Entry entr
                 if (unit == 256 && same && (256 - e) % 256 < t.numel)
                     ok = ok && check(h == (256 - e) % 256, "a one-wave kernel's units do not start at whole units", &l);
             }
-            const uint64_t u = (t.numel - (D.vec ? D.head : 0) + unit - 1) / unit;
+            const uint64_t u = (t.numel - (D.vec ? D.head() : 0) + unit - 1) / unit;
             ok = ok && check(D.unit_begin == units, "units are not the kernel's", &l);
             units += u;
             elems += t.numel;
