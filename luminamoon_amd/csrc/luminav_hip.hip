@@ -591,8 +591,8 @@ static int launch(const Kernel &kernel, Args &args, int mode, int pt, int st, in
     // at 1e9 and 3.5e9 elements and 2% faster at 6.7e9; 16-bit-state launches ran level to 4.6%
     // slower. Results are the same either way: units are independent and the count is exact in
     // any order.
-    // The fused radial step in f32 with the reference defaults maps b to b too. Against the other mapping, in one
-    // process, lists of 20 tensors and buckets of 3e5-6e8 elements: CLM and T2 with their limit of 5 blocks per
+    // The fused radial step in f32 with the reference defaults maps b to b too. Speeds against the other mapping,
+    // in one process, lists of 20 tensors and buckets of 3e5-6e8 elements: CLM and T2 with their limit of 5 blocks per
     // CU (below) 0.97-1.15x, mean 1.05x, slowest at 8e6 (0.97x, buckets) and 1.8e8-3e8 (0.97x, CLM lists).
     // TD-CLM and T1 up to 2^17 units 0.94-1.10x, mean 1.02x (1.02-1.10x at 2e6 and 1.2e7-2.4e7, 0.94-1.05x
     // at 5e7-1.3e8); above it 0.93-1.04x, mean 0.99x, so there they keep the other mapping. The other radial

@@ -178,7 +178,7 @@ constexpr uint32_t wave_resident(int mode, int pt, bool master) {
 // Whether the large form of a table launch runs one-wave blocks too. The applying and single passes do; a
 // fused pass also reports its counts. A table launch has the count slots of 1024-element units (the
 // workspace is sized for those), so up to 256 one-wave blocks report to one slot, and atomics of several
-// XCDs on one line take turns: 50-500 tensors of 1.3e6 elements or less ran 0.75-1.0x of 256-thread blocks,
+// XCDs on one line take turns. Speeds against 256-thread blocks: 50-500 tensors of 1.3e6 elements or less 0.75-1.0x,
 // with 64 blocks per slot 0.93-1.07x, without reports 0.95-1.08x (four slots to a line are as slow as
 // one). Fused one-wave blocks pay for that only where a limit on them gains more: not at 32 per CU, where
 // 256-thread blocks of the same lanes are as fast (f32 state, 60 and 400 tensors and two models,
@@ -189,8 +189,8 @@ constexpr bool wave_table(int mode, int pt, int pass, bool master) {
 }
 
 // Smallest mean tensor of a one-wave table launch, in elements: larger tensors have the most count slots
-// either way, and finish a slot's blocks over a longer time. Fused steps against 256-thread blocks, ragged
-// lists of 60-400 tensors and GPT-2 and Llama shapes, by mean tensor:
+// either way, and finish a slot's blocks over a longer time. Speeds against 256-thread blocks of fused steps
+// over ragged lists of 60-400 tensors and GPT-2 and Llama shapes, by mean tensor:
 //   28 bytes an element (CLM, T2: f32, or with a master)   0.35-0.9e6: 0.93-1.08x   1.1e6 and up: 1.00-1.13x
 //   20-22 bytes                                             0.35-0.9e6: 0.80-1.08x   1.1-1.9e6: 0.94-1.09x
 //                                                           2.2e6 and up: 0.96-1.06x (means 1.01-1.05x)
